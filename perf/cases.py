@@ -50,32 +50,32 @@ def _advance(name, mech, n, api="update", host=False, carried=False, flow=0, int
 def listed():
     return [
         # a reactor calculation or a small test: host arrays, one wavefront of cells
-        _advance("h2air step, 64 cells, host", "h2air", 64, host=True),
+        _advance("h2air step 64 host", "h2air", 64, host=True),
         # a 65,536-cell domain: source terms for the flow solver, first step
-        _advance("h2air source step, 64k", "h2air", 65536, api="solve"),
+        _advance("h2air source step 64k", "h2air", 65536, api="solve"),
         # a 1M-cell domain mid-run: sub-step memory and schedule of the step before
-        _advance("h2air step, 1M, carried", "h2air", 1 << 20, carried=True),
+        _advance("h2air step 1M carried", "h2air", 1 << 20, carried=True),
         # a larger mechanism on a small ragged domain
-        _advance("syn32 source step, 4099", "syn32", 4099, api="solve"),
+        _advance("syn32 source step 4099", "syn32", 4099, api="solve"),
         # a larger mechanism on a large domain mid-run (the headline benchmark's kernel)
-        _advance("syn32 step, 512k, carried", "syn32", 1 << 19, carried=True),
+        _advance("syn32 step 512k carried", "syn32", 1 << 19, carried=True),
         # the largest benchmark mechanism
-        _advance("syn54 step, 48k", "syn54", 49152),
+        _advance("syn54 step 48k", "syn54", 49152),
         # transport of a large domain, every flow step
-        {"name": "h2air props, 1M", "kind": "props", "mech": "h2air", "n": 1 << 20, "precision": 0},
+        {"name": "h2air props 1M", "kind": "props", "mech": "h2air", "n": 1 << 20, "precision": 0},
         # transport with a larger mechanism on a ragged domain
-        {"name": "syn32 props, 262147", "kind": "props", "mech": "syn32", "n": 262147,
+        {"name": "syn32 props 262147", "kind": "props", "mech": "syn32", "n": 262147,
          "precision": 0},
         # temperature recovery of every cell after a transport step
-        {"name": "syn32 T from h, 1M", "kind": "T_from_h", "mech": "syn32", "n": 1 << 20,
+        {"name": "syn32 T from h 1M", "kind": "T_from_h", "mech": "syn32", "n": 1 << 20,
          "energy": False},
         # point-implicit coupling of the chemistry source
-        {"name": "syn32 source diag, 256k", "kind": "source", "mech": "syn32", "n": 1 << 18},
+        {"name": "syn32 source diag 256k", "kind": "source", "mech": "syn32", "n": 1 << 18},
         # one mini-batch of surrogate training at the trainer's default batch
-        {"name": "surrogate gradient, 16384", "kind": "train", "mech": "syn32", "n": 16384,
+        {"name": "surrogate gradient 16384", "kind": "train", "mech": "syn32", "n": 16384,
          "width": 256},
         # network evaluation of a field
-        {"name": "surrogate predict, 1M", "kind": "predict", "mech": "syn32", "n": 1 << 20,
+        {"name": "surrogate predict 1M", "kind": "predict", "mech": "syn32", "n": 1 << 20,
          "width": 256, "precision": 0},
     ]
 
