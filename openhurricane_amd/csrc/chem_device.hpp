@@ -62,6 +62,28 @@ constexpr double csqrt(double x) {
     return r;
 }
 
+// compile-time x^p for a positive constant x (mantissa and exponent split, the
+// logarithm's atanh series and the exponential's Taylor series to the last bit
+// that changes the sum)
+constexpr double cpow_const(double x, double p) {
+    constexpr double kLn2 = 0.69314718055994530942;
+    int e = 0;
+    while (x > 1.5) { x *= 0.5; ++e; }
+    while (x < 0.75) { x *= 2.0; --e; }
+    const double z = (x - 1.0) / (x + 1.0), z2 = z * z;
+    double ln = 0.0, t = z;
+    for (int n = 1; n < 60; n += 2, t *= z2) ln += t / n;
+    double y = p * (2.0 * ln + e * kLn2);
+    int k = 0;
+    while (y > 0.5 * kLn2) { y -= kLn2; ++k; }
+    while (y < -0.5 * kLn2) { y += kLn2; --k; }
+    double r = 1.0, u = 1.0;
+    for (int n = 1; n < 30; ++n) r += (u *= y / n);
+    for (; k > 0; --k) r *= 2.0;
+    for (; k < 0; ++k) r *= 0.5;
+    return r;
+}
+
 template <int B, int E, class F>
 __device__ __forceinline__ void sfor(F &&f) {
     if constexpr (B < E) {
@@ -83,6 +105,14 @@ __device__ __forceinline__ double frcp(double x) {
     r = fma(e, r, r);
     e = fma(-x, r, 1.0);
     return fma(e, r, r);
+}
+
+// refined 1/sqrt(x), x normal and positive
+__device__ __forceinline__ double frsq(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    const double hx = 0.5 * x;
+    r = fma(r, fma(-hx * r, r, 0.5), r);
+    return fma(r, fma(-hx * r, r, 0.5), r);
 }
 
 // x^p for a compile-time exponent p >= 0 (integer exponents as products).
@@ -135,6 +165,27 @@ constexpr double tcommon_max() {
     double v = M::Tcommon[0];
     for (int k = 1; k < M::NS; ++k) v = M::Tcommon[k] > v ? M::Tcommon[k] : v;
     return v;
+}
+
+// Temperatures that every species' fit covers, and whether one Tcommon
+// splits them all.
+template <class M>
+constexpr double tlow_max() {
+    double v = M::Tlow[0];
+    for (int k = 1; k < M::NS; ++k) v = M::Tlow[k] > v ? M::Tlow[k] : v;
+    return v;
+}
+template <class M>
+constexpr double thigh_min() {
+    double v = M::Thigh[0];
+    for (int k = 1; k < M::NS; ++k) v = M::Thigh[k] < v ? M::Thigh[k] : v;
+    return v;
+}
+template <class M>
+constexpr bool uniform_tcommon() {
+    for (int k = 1; k < M::NS; ++k)
+        if (M::Tcommon[k] != M::Tcommon[0]) return false;
+    return true;
 }
 
 // Whether every active lane of the wavefront is at or above every Tcommon

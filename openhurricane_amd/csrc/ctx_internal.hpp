@@ -12,6 +12,7 @@
 #include "../../include/ohc.h"
 #include "lane_kernels.hpp"
 #include "mech.hpp"
+#include "wave_dispatch.hpp"
 #include "wave_kernels.hpp"
 
 struct ohc_mech {
@@ -29,6 +30,7 @@ struct ohc_ctx {
     bool wave = false;          // generic wavefront-per-cell kernels (run-time tables)
     ohcd::WMech wm{};           // device tables of the generic kernels
     void *d_wm = nullptr;       // one allocation holding them
+    ohcd::PairTab pair{};       // pair constants of the mixture rules (in d_wm)
     int grid = 0;  // persistent integrator grid (single-wavefront blocks)
     int cus = 0;         // compute units of the device
     int max_per_cu = 0;  // resident integrator blocks per CU the kernel allows

@@ -104,7 +104,8 @@ int ensure_sched(ohc_ctx *c, int64_t n) {
 // Device tables of the generic kernels: species fields [field][64], reaction
 // fields chunk-major [nrp / 64][field][64] (the 64 reactions a wavefront
 // evaluates at once, field by field) -- a packed 32-bit table read for every
-// reaction and an FP64 table -- and efficiencies [nr][64].
+// reaction and an FP64 table -- and efficiencies by reaction [nr][64] and
+// transposed within each chunk.
 int build_wmech(ohc_ctx *c) {
     using namespace ohcd;
     const ohc::Mechanism &m = c->mech;
@@ -148,6 +149,39 @@ int build_wmech(ohc_ctx *c) {
             for (int i = 0; i < 4; ++i) sp[(og + i) * 64 + k] = gq[i];
         }
     }
+    // derived species constants and pair constants of the mixture rules
+    // (kineticTheory.cpp:37-168, transportList.cpp:309-333)
+    for (int k = 0; k < 64; ++k) {
+        const double W = sp[SP_W * 64 + k], ek = sp[SP_EKB * 64 + k], sg = sp[SP_SIG * 64 + k];
+        sp[SP_IW * 64 + k] = 1.0 / W;
+        sp[SP_IEK * 64 + k] = 1.0 / ek;
+        sp[SP_OMC * 64 + k] = 1.147 * std::pow(ek, 0.145);
+        sp[SP_MUC * 64 + k] = 2.6693e-6 * std::sqrt(W) / (sg * sg);
+        sp[SP_W4 * 64 + k] = 1.0 / std::sqrt(std::sqrt(W));
+        sp[SP_IW4 * 64 + k] = std::sqrt(std::sqrt(W));
+        sp[SP_SQW * 64 + k] = std::sqrt(W);
+    }
+    std::vector<double> pair((size_t)64 * PairTab::kRow, 0.0);
+    for (int i = 0; i < ns; ++i)
+        for (int j = 0; j < ns; ++j) {
+            double *t = &pair[(size_t)i * PairTab::kRow + (j / 8) * 32 + j % 8];
+            const double Wi = sp[SP_W * 64 + i], Wj = sp[SP_W * 64 + j];
+            const double sij = 0.5 * (sp[SP_SIG * 64 + i] + sp[SP_SIG * 64 + j]);
+            const double ek = std::sqrt(sp[SP_EKB * 64 + i] * sp[SP_EKB * 64 + j]);
+            const double cst = 1.858e-7 * std::sqrt(1.0 / Wi + 1.0 / Wj) / (sij * sij) * kPatm;
+            t[0] = 1.0 / std::sqrt(8.0) / std::sqrt(1.0 + Wi / Wj);
+            t[8] = i == j ? 0.0 : std::pow(ek, 0.145) / cst;
+            t[16] = 1.0 / ek;
+            t[24] = i == j ? 0.0 : 1.0 / cst;
+        }
+    c->wm.uniform_range = 1;
+    c->wm.Tmin = 0.0;
+    c->wm.Tmax = 1.0e300;
+    for (int k = 0; k < ns; ++k) {
+        if (m.Tcommon[k] != m.Tcommon[0]) c->wm.uniform_range = 0;
+        c->wm.Tmin = std::max(c->wm.Tmin, (double)m.Tlow[k]);
+        c->wm.Tmax = std::min(c->wm.Tmax, (double)m.Thigh[k]);
+    }
     // Table slot q holds reaction perm[q]: reactions grouped by rate type,
     // reversibility and fall-off form (stable, so file order within a group),
     // so that a 64-reaction chunk of the wavefront mostly takes one code path.
@@ -167,7 +201,8 @@ int build_wmech(ohc_ctx *c) {
         return u;
     };
     std::vector<uint32_t> rh((size_t)RH_NFIELD * nrp, 0u);
-    std::vector<double> rd((size_t)RD_NFIELD * nrp, 0.0), eff((size_t)std::max(nr, 1) * 64, 0.0);
+    std::vector<double> rd((size_t)RD_NFIELD * nrp, 0.0), eff((size_t)std::max(nr, 1) * 64, 0.0),
+        efft((size_t)nrp * 64, 0.0);
     for (int q = 0; q < nr; ++q) {
         const int r = perm[q];
         double s = 0.0;
@@ -207,13 +242,17 @@ int build_wmech(ohc_ctx *c) {
         }
         for (int i = 0; i < 5; ++i) rd[xd(RD_FOP + i, q)] = m.fo[5 * r + i];
         if (m.kind[r] != OHC_RATE_ARRHENIUS)
-            for (int k = 0; k < ns; ++k) eff[(size_t)q * 64 + k] = m.eff[(size_t)r * ns + k];
+            for (int k = 0; k < ns; ++k) {
+                eff[(size_t)q * 64 + k] = m.eff[(size_t)r * ns + k];
+                efft[((size_t)(q / 64) * 64 + k) * 64 + q % 64] = m.eff[(size_t)r * ns + k];
+            }
     }
     // one device allocation, 256-byte aligned pieces
     auto al = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t b_sp = al(sp.size() * 8), b_rh = al(rh.size() * 4), b_rd = al(rd.size() * 8),
-                 b_ef = al(eff.size() * 8);
-    const size_t total = b_sp + b_rh + b_rd + b_ef;
+                 b_ef = al(eff.size() * 8), b_et = al(efft.size() * 8),
+                 b_pr = al(pair.size() * 8);
+    const size_t total = b_sp + b_rh + b_rd + b_ef + b_et + b_pr;
     std::vector<unsigned char> h(total, 0);
     size_t off = 0;
     auto put = [&](const void *src, size_t bytes, size_t span) {
@@ -223,7 +262,9 @@ int build_wmech(ohc_ctx *c) {
         return o;
     };
     const size_t o_sp = put(sp.data(), sp.size() * 8, b_sp), o_rh = put(rh.data(), rh.size() * 4, b_rh),
-                 o_rd = put(rd.data(), rd.size() * 8, b_rd), o_ef = put(eff.data(), eff.size() * 8, b_ef);
+                 o_rd = put(rd.data(), rd.size() * 8, b_rd), o_ef = put(eff.data(), eff.size() * 8, b_ef),
+                 o_et = put(efft.data(), efft.size() * 8, b_et),
+                 o_pr = put(pair.data(), pair.size() * 8, b_pr);
     HIPCHK(c, hipMalloc(&c->d_wm, total));
     HIPCHK(c, hipMemcpy(c->d_wm, h.data(), total, hipMemcpyHostToDevice));
     unsigned char *d = (unsigned char *)c->d_wm;
@@ -234,6 +275,8 @@ int build_wmech(ohc_ctx *c) {
     c->wm.rh = (const unsigned *)(d + o_rh);
     c->wm.rd = (const double *)(d + o_rd);
     c->wm.eff = (const double *)(d + o_ef);
+    c->wm.efft = (const double *)(d + o_et);
+    c->pair.t = (const double *)(d + o_pr);
     return OHC_OK;
 }
 
@@ -277,7 +320,8 @@ hipError_t launch_integrator(const ohc_ctx *c, const ohcd::LaneParams &P) {
     W.L = P;
     W.M = c->wm;
     W.exact_dkp = c->opts.jacobian;
-    const int grid = (int)std::min<int64_t>(c->grid, P.n);
+    const int per = ohcd::wave_cells(c->mech.ns + 1, P.integrator);
+    const int grid = (int)std::min<int64_t>(c->grid, (P.n + per - 1) / per);
     return ohcd::wave_integrate(W, grid, c->stream);
 }
 
@@ -589,7 +633,7 @@ int ohc_ctx_create(const ohc_mech *m, const ohc_opts *opts, int32_t device, ohc_
         hipDeviceProp_t prop;
         HIPCHK(cp, hipGetDeviceProperties(&prop, device));
         int per_cu = 0;
-        const void *fn = c->lane ? c->lane->integrate_fn : ohcd::wave_integrate_fn(c->mech.ns + 1);
+        const void *fn = c->lane ? c->lane->integrate_fn : ohcd::wave_integrate_fn(c->mech.ns + 1, o.integrator);
         HIPCHK(cp, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64, 0));
         c->cus = prop.multiProcessorCount;
         c->max_per_cu = std::max(per_cu, 1);
@@ -966,7 +1010,8 @@ static int mix_common(ohc_ctx *c, int64_t n, const double *T, const double *p, c
                        ldD,        (double *)dcp,      (double *)dha,      (double *)dhk,
                        c->opts.precision, (double *)dcv, (double *)dea};
     if (c->lane) HIPCHK(c, c->lane->props(P, c->stream));
-    else HIPCHK(c, ohcd::wave_props(P, c->wm, c->stream));
+    else if (P.prec == 1) HIPCHK(c, ohcd::wave_props(P, c->wm, c->stream));
+    else HIPCHK(c, ohcd::table_props(P, c->wm, c->pair, c->stream));
     return st.finish();
 }
 

@@ -3,6 +3,7 @@
 // unit (wave_size.hip compiled with -DOHC_WAVE_N=N), so they build in parallel.
 #include "wave_dispatch.hpp"
 
+#include "quad_kernels.hpp"
 #include "wave_kernels.hpp"
 
 namespace ohcd {
@@ -13,7 +14,7 @@ namespace ohcd {
     hipError_t wave_source_##n(const SourceParams &, const WMech &, hipStream_t);    \
     hipError_t wave_kim_##n(const KimParams &, const WMech &, int, hipStream_t);     \
     hipError_t wave_lu_##n(const LuParams &, hipStream_t);                           \
-    const void *wave_fn_##n();
+    const void *wave_fn_##n(int);
 OHC_WAVE_DECL(12)
 OHC_WAVE_DECL(16)
 OHC_WAVE_DECL(24)
@@ -32,7 +33,7 @@ struct Entry {
     hipError_t (*source)(const SourceParams &, const WMech &, hipStream_t);
     hipError_t (*kim)(const KimParams &, const WMech &, int, hipStream_t);
     hipError_t (*lu)(const LuParams &, hipStream_t);
-    const void *(*fn)();
+    const void *(*fn)(int);
 };
 
 #define OHC_WAVE(n) \
@@ -79,16 +80,18 @@ hipError_t wave_lu(const LuParams &p, hipStream_t s) {
     return e ? e->lu(p, s) : hipErrorInvalidValue;
 }
 
-// ---- mixture thermo + transport for run-time tables ----------------------
+// ---- mixture thermo + transport for run-time tables, split precision -----
 // One wavefront per cell, species k in lane k; the mixture rules are wavefront
 // reductions (wsum) and the pair sums of Wilke's rule and of the
 // mixture-averaged diffusivities run in lane i over j with the other
 // species' values broadcast from LDS.  Same formulas as props_lane_kernel
 // (JANAF.cpp:155-189, speciesList.cpp:208-222, kineticTheory.cpp:37-168,
-// kineticTheory.inl:32-34, transportList.cpp:309-333).  F = double: FP64;
-// F = float (split precision): the kinetic-theory species properties,
-// Wilke's rule and the binary / mixture-averaged diffusivities in FP32, the
-// thermo, mole fractions and wavefront sums in FP64.
+// kineticTheory.inl:32-34, transportList.cpp:309-333).  F = float: the
+// kinetic-theory species properties, Wilke's rule and the binary /
+// mixture-averaged diffusivities in FP32, the thermo, mole fractions and
+// wavefront sums in FP64.  (The FP64 mode runs on props_table.hip, which
+// regroups the pair terms; in FP32 that would change results by FP32
+// rounding.)
 constexpr int kPropWaves = 4;  // cells (wavefronts) per 256-thread block
 
 template <class F>
@@ -194,70 +197,20 @@ __global__ __launch_bounds__(256) void props_wave_kernel(const PropParams P, con
     }
 }
 
-// thermoList::T (thermoList.cpp:504-533) for run-time tables: one lane per
-// cell, species loop over the table (uniform addresses across the lanes).
-__global__ __launch_bounds__(256) void tfromh_table_kernel(const ThParams P, const WMech M) {
-    const int64_t cell = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (cell >= P.n) return;
-    const double hstar = P.h[cell];
-    const double T0 = P.T[cell], Ttol = T0 * 1.0e-4;
-    double Rm = 0.0;
-    if (P.energy) {  // TEa: F = ha - Rm T, dF/dT = cp - Rm (thermoList.inl:343-370)
-        double s = 0.0;
-        for (int k = 0; k < M.ns; ++k) s += P.Y[k * P.ldY + cell] / M.sp[SP_W * 64 + k];
-        Rm = kRu / (M.ns == 1 ? M.sp[SP_W * 64] : 1.0 / fmax(s, kVeryTiny));
-    }
-    double Test = T0, Tnew = T0;
-    int iter = 0, flag = 1;
-    do {
-        Test = Tnew;
-        const TFac tf = tfac(Test);
-        double hm = 0.0, cpm = 0.0;
-        for (int k = 0; k < M.ns; ++k) {
-            double G, dG, Cp, H, dCp;
-            wthermo(M, k, tf, G, dG, Cp, H, dCp);
-            const double W = M.sp[SP_W * 64 + k], yk = P.Y[k * P.ldY + cell];
-            hm += H / W * yk;
-            cpm += Cp / W * yk;
-        }
-        if (P.energy) {
-            hm -= Rm * Test;
-            cpm -= Rm;
-        }
-        double Tn = Test - (hm - hstar) / cpm;
-        if (Tn < P.Tlow) {
-            flag = 0;
-            Tn = P.Tlow;
-        } else if (Tn > P.Thigh) {
-            flag = 2;
-            Tn = P.Thigh;
-        } else {
-            flag = 1;
-        }
-        Tnew = Tn;
-        if (iter++ > 100) break;
-    } while (fabs(Tnew - Test) > Ttol);
-    P.T[cell] = Tnew;
-    if (P.iflag) P.iflag[cell] = flag;
-}
-
 hipError_t wave_props(const PropParams &p, const WMech &m, hipStream_t s) {
     const unsigned grid = (unsigned)((p.n + kPropWaves - 1) / kPropWaves);
-    if (p.prec == 1)
-        hipLaunchKernelGGL(props_wave_kernel<float>, dim3(grid), dim3(64 * kPropWaves), 0, s, p, m);
-    else
-        hipLaunchKernelGGL(props_wave_kernel<double>, dim3(grid), dim3(64 * kPropWaves), 0, s, p, m);
+    hipLaunchKernelGGL(props_wave_kernel<float>, dim3(grid), dim3(64 * kPropWaves), 0, s, p, m);
     return hipGetLastError();
 }
 
-hipError_t wave_tfromh(const ThParams &p, const WMech &m, hipStream_t s) {
-    hipLaunchKernelGGL(tfromh_table_kernel, dim3((unsigned)((p.n + 255) / 256)), dim3(256), 0, s, p, m);
-    return hipGetLastError();
-}
-
-const void *wave_integrate_fn(int n) {
+const void *wave_integrate_fn(int n, int integrator) {
     const Entry *e = pick(n);
-    return e ? e->fn() : nullptr;
+    return e ? e->fn(integrator) : nullptr;
+}
+
+int wave_cells(int n, int integrator) {
+    const Entry *e = pick(n);
+    return e && e->N <= kQuadMaxN && integrator == 0 ? 4 : 1;
 }
 
 }  // namespace ohcd

@@ -57,6 +57,13 @@ enum {
     SP_GHI = SP_GLO + 4,
     SP_EKB = SP_GHI + 4,  // transport: eps/k [K]
     SP_SIG,               // transport: sigma [Angstrom]
+    SP_IW,                // 1 / W
+    SP_IEK,               // k / eps
+    SP_OMC,               // 1.147 (eps / k)^0.145: the power term of Omega22 over T^-0.145
+    SP_MUC,               // 2.6693e-6 sqrt(W) / sigma^2
+    SP_W4,                // W^(-1/4)
+    SP_IW4,               // W^(1/4)
+    SP_SQW,               // W^(1/2)
     SP_NFIELD
 };
 // Reaction tables are chunk-major: reaction r = 64 c + l (the chunk a
@@ -100,6 +107,11 @@ struct WMech {
     const unsigned *rh;   // [nrp / 64][RH_NFIELD][64]
     const double *rd;     // [nrp / 64][RD_NFIELD][64]
     const double *eff;    // [nr][64] third-body efficiencies
+    const double *efft;   // [nrp / 64][64 species][64 reactions]: the same, lane-contiguous
+    // one Tcommon for all species and the temperatures every species' fit
+    // covers (props_table.hip)
+    int uniform_range;
+    double Tmin, Tmax;
 };
 
 struct WaveParams {
@@ -112,7 +124,7 @@ struct WaveParams {
 // the one vector offset, the chunk and field a scalar offset, so a table read
 // needs no vector address arithmetic.  Reads past a table return zero.
 struct RxnTab {
-    __amdgpu_buffer_rsrc_t rh, rd, ef;
+    __amdgpu_buffer_rsrc_t rh, rd, ef, et;
 };
 __device__ __forceinline__ RxnTab rxn_tab(const WMech &M) {
     constexpr int kRsrcWord3 = 0x00020000;  // raw 32-bit data, CDNA
@@ -120,6 +132,7 @@ __device__ __forceinline__ RxnTab rxn_tab(const WMech &M) {
     t.rh = __builtin_amdgcn_make_buffer_rsrc((void *)M.rh, 0, RH_NFIELD * M.nrp * 4, kRsrcWord3);
     t.rd = __builtin_amdgcn_make_buffer_rsrc((void *)M.rd, 0, RD_NFIELD * M.nrp * 8, kRsrcWord3);
     t.ef = __builtin_amdgcn_make_buffer_rsrc((void *)M.eff, 0, M.nr * 64 * 8, kRsrcWord3);
+    t.et = __builtin_amdgcn_make_buffer_rsrc((void *)M.efft, 0, M.nrp * 64 * 8, kRsrcWord3);
     return t;
 }
 // field f of reaction 64 c + lane (c wave-uniform)
@@ -133,9 +146,10 @@ __device__ __forceinline__ double ldd(const RxnTab &t, int f, int c, int lane) {
     return __builtin_bit_cast(
         double, __builtin_amdgcn_raw_buffer_load_b64(t.rd, lane * 8, (c * RD_NFIELD + f) * 512, 0));
 }
-// efficiency of species k (wave-uniform) in reaction r
-__device__ __forceinline__ double lde(const RxnTab &t, int r, int k) {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(t.ef, r * 512, k * 8, 0));
+// efficiency of species k (wave-uniform) in reaction 64 c + lane
+__device__ __forceinline__ double lde(const RxnTab &t, int c, int lane, int k) {
+    return __builtin_bit_cast(
+        double, __builtin_amdgcn_raw_buffer_load_b64(t.et, lane * 8, (c * 64 + k) * 512, 0));
 }
 // efficiency of species `lane` in reaction r (wave-uniform)
 __device__ __forceinline__ double lde_col(const RxnTab &t, int r, int lane) {
@@ -368,12 +382,13 @@ struct WRxn {
 // F = float: the split-precision mode -- Arrhenius rate constants and the
 // equilibrium constant (Gibbs sums and exponential) in FP32; concentration
 // products, rates, derivatives in FP64.
+// Reaction 64 ch + lane of the tables (ch wave-uniform); sc, sG, sdG: the
+// cell's concentrations, G and dG/dT by species in LDS.
 template <bool WITH_J, class FT = double>
-__device__ __forceinline__ void wreaction(const WMech &M, int base, const TFac &tf,
+__device__ __forceinline__ void wreaction(const WMech &M, int ch, int lane, const TFac &tf,
                                           const double *sc, const double *sG, const double *sdG,
                                           int exact, WRxn &o) {
     const RxnTab tb = rxn_tab(M);
-    const int lane = threadIdx.x, ch = base >> 6, r = base + lane;
     const unsigned hdr = ldu(tb, RH_HDR, ch, lane), ix = ldu(tb, RH_IDX, ch, lane),
                    ix2 = ldu(tb, RH_IDX2, ch, lane);
     const int nf = hdr & 3u, nb = (hdr >> 2) & 3u, rev = (hdr >> 4) & 3u, kind = (hdr >> 6) & 7u;
@@ -408,7 +423,7 @@ __device__ __forceinline__ void wreaction(const WMech &M, int base, const TFac &
     double Mtb = 0.0;
     if (kind != 0) {
 #pragma unroll 8
-        for (int k = 0; k < M.ns; ++k) Mtb += lde(tb, r, k) * sc[k];
+        for (int k = 0; k < M.ns; ++k) Mtb += lde(tb, ch, lane, k) * sc[k];
     }
     double kf, k0 = 0.0, kinf = 0.0, Pr = 0.0, F = 1.0;
     FoState fs{1.0, 0.0, 0.0};
@@ -621,7 +636,7 @@ __device__ __forceinline__ double wave_eval(const WMech &M, WaveLDS<N> &L, doubl
         WRxn o;
         o.nf = o.nb = 0;
         if (r < M.nr) {
-            wreaction<WITH_J, F>(M, base, tf, L.c, L.G, L.dG, exact, o);
+            wreaction<WITH_J, F>(M, base >> 6, lane, tf, L.c, L.G, L.dG, exact, o);
             // d(omega)/dt rows of the participants: sigma_a q, and with J the
             // row terms sigma_a dq/dc_j and sigma_a dq/dT
 #pragma unroll
@@ -1210,7 +1225,7 @@ __device__ __forceinline__ double wave_mts_diag(const WMech &M, WaveLDS<N> &L, d
         const int r = base + lane;
         if (r < M.nr) {
             WRxn o;
-            wreaction<true>(M, base, tf, L.c, L.G, L.dG, exact, o);
+            wreaction<true>(M, base >> 6, lane, tf, L.c, L.G, L.dG, exact, o);
 #pragma unroll
             for (int i = 0; i < kWP; ++i) {
                 if (i < o.nf) {
@@ -1436,7 +1451,7 @@ __global__ __launch_bounds__(64) void kim_wave_kernel(const KimParams P, const W
         const int r = base + lane;
         if (r < M.nr) {
             WRxn o;
-            wreaction<true>(M, base, tf, L.c, L.G, L.dG, P.exact, o);
+            wreaction<true>(M, base >> 6, lane, tf, L.c, L.G, L.dG, P.exact, o);
 #pragma unroll
             for (int i = 0; i < kWP; ++i) {
                 if (i < o.nf) lds_add(&L.w[o.fi[i]], -o.fnu[i] * o.q);

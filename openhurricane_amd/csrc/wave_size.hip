@@ -1,5 +1,6 @@
 // wave_size.hip -- the generic kernels for one padded ODE size OHC_WAVE_N
 // (compiled once per size; see wave_dispatch.hip).
+#include "quad_kernels.hpp"
 #include "wave_kernels.hpp"
 
 #ifndef OHC_WAVE_N
@@ -10,6 +11,16 @@
 #define OHC_CAT(a, b) OHC_CAT2(a, b)
 
 namespace ohcd {
+
+// ImplicitEuler: four cells per wavefront up to kQuadMaxN unknowns, one above
+// (a lane would hold more rows of the system than its registers).
+template <int N, int FLOW, class F>
+static void launch_ie(const WaveParams &p, int grid, hipStream_t s) {
+    if constexpr (N <= kQuadMaxN)
+        hipLaunchKernelGGL((ie_quad_kernel<N, FLOW, F>), dim3(grid), dim3(64), 0, s, p);
+    else
+        hipLaunchKernelGGL((ie_wave_kernel<N, FLOW, 0, F>), dim3(grid), dim3(64), 0, s, p);
+}
 
 hipError_t OHC_CAT(wave_integrate_, OHC_WAVE_N)(const WaveParams &p, int grid, hipStream_t s) {
     constexpr int N = OHC_WAVE_N;
@@ -23,12 +34,12 @@ hipError_t OHC_CAT(wave_integrate_, OHC_WAVE_N)(const WaveParams &p, int grid, h
         if (p.L.flow == 0) hipLaunchKernelGGL((ie_wave_kernel<N, 0, 2>), dim3(grid), dim3(64), 0, s, p);
         else hipLaunchKernelGGL((ie_wave_kernel<N, 1, 2>), dim3(grid), dim3(64), 0, s, p);
     } else if (p.L.prec == 1) {
-        if (p.L.flow == 0) hipLaunchKernelGGL((ie_wave_kernel<N, 0, 0, float>), dim3(grid), dim3(64), 0, s, p);
-        else hipLaunchKernelGGL((ie_wave_kernel<N, 1, 0, float>), dim3(grid), dim3(64), 0, s, p);
+        if (p.L.flow == 0) launch_ie<N, 0, float>(p, grid, s);
+        else launch_ie<N, 1, float>(p, grid, s);
     } else if (p.L.flow == 0) {
-        hipLaunchKernelGGL((ie_wave_kernel<N, 0>), dim3(grid), dim3(64), 0, s, p);
+        launch_ie<N, 0, double>(p, grid, s);
     } else {
-        hipLaunchKernelGGL((ie_wave_kernel<N, 1>), dim3(grid), dim3(64), 0, s, p);
+        launch_ie<N, 1, double>(p, grid, s);
     }
     return hipGetLastError();
 }
@@ -67,8 +78,14 @@ hipError_t OHC_CAT(wave_lu_, OHC_WAVE_N)(const LuParams &p, hipStream_t s) {
     return hipGetLastError();
 }
 
-const void *OHC_CAT(wave_fn_, OHC_WAVE_N)() {
-    return (const void *)&ie_wave_kernel<OHC_WAVE_N, 0>;
+const void *OHC_CAT(wave_fn_, OHC_WAVE_N)(int integrator) {
+    constexpr int N = OHC_WAVE_N;
+    if constexpr (N <= kQuadMaxN) {
+        if (integrator == 0) return (const void *)&ie_quad_kernel<N, 0>;
+        return (const void *)&ie_wave_kernel<N, 0, 2>;
+    } else {
+        return (const void *)&ie_wave_kernel<N, 0>;
+    }
 }
 
 }  // namespace ohcd
