@@ -230,7 +230,14 @@ int build_wmech(ohc_ctx *c) {
         }
         rd[xd(RD_SUMS, q)] = s;
         put_f(RH_SUMS, s);
-        rh[xh(RH_HDR, q)] = (uint32_t)m.nf[r] | (uint32_t)m.nb[r] << 2 | (uint32_t)m.rev[r] << 4 |
+        uint32_t ord = 0;
+        for (int i = 0; i < kWP; ++i) {
+            const double fo = i < m.nf[r] ? m.f_ord[r * P + i] : 1.0;
+            const double bo = i < m.nb[r] ? m.b_ord[r * P + i] : 1.0;
+            ord |= (fo == 2.0 ? 1u << (kRhSq + i) : 0u) | (bo == 2.0 ? 1u << (kRhSq + kWP + i) : 0u);
+            if ((fo != 1.0 && fo != 2.0) || (bo != 1.0 && bo != 2.0)) ord |= kRhPow;
+        }
+        rh[xh(RH_HDR, q)] = ord | (uint32_t)m.nf[r] | (uint32_t)m.nb[r] << 2 | (uint32_t)m.rev[r] << 4 |
                             (uint32_t)m.kind[r] << 6 | (uint32_t)m.fo_type[r] << 9 |
                             (gen ? kRhGen : 0u);
         rh[xh(RH_IDX, q)] = fidx[0] | fidx[1] << 8 | fidx[2] << 16 | bidx[0] << 24;

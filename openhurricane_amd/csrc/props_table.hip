@@ -51,11 +51,15 @@ __device__ __forceinline__ void species_cp_h(ctab *S, int k, double T, double &c
 }
 
 template <int NSP>
-__global__ __launch_bounds__(64) void props_table_kernel(const PropParams P, const WMech M,
+__global__ __launch_bounds__(64, NSP <= 32 ? 3 : 1) void props_table_kernel(const PropParams P, const WMech M,
                                                          const PairTab pt) {
     // up to 32 species x, x b and x b^2 fit the registers; above, x and b, with
     // one more multiplication per pair
-    constexpr bool kThree = NSP <= 32;
+    // x, x b and x b^2 in registers up to 16 species; above, x and b, with one
+    // more multiplication per pair, so that three wavefronts share a SIMD and hide the
+    // scalar loads of the rows (32 species, 262,147 cells: 514 us with x, x b, x b^2
+    // at one wavefront, 385 us so)
+    constexpr bool kThree = NSP <= 16;
     __shared__ double s_a[NSP][64];
     const int lane = threadIdx.x, ns = M.ns;
     const int64_t c0 = (int64_t)blockIdx.x * 64;

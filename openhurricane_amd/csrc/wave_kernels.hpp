@@ -31,14 +31,6 @@ namespace ohcd {
 
 constexpr int kWP = 3;  // distinct species per reaction side in the run-time tables
 
-// How the LU's pivot row reaches the other lanes: 1 by v_readlane pairs (two
-// vector ALU instructions per element, no LDS round trip), 2 by ds_bpermute
-// pairs (no vector ALU work, but an LDS round trip on every step's critical
-// path: 1.3x the LU time of 1 on the 32-species mechanism), 0 through an LDS
-// row buffer written by the pivot lane (a barrier per elimination step).
-#ifndef OHC_LU_BCAST
-#define OHC_LU_BCAST 1
-#endif
 static_assert(kWP == 3, "the reaction kernels multiply three participant powers");
 
 // species fields, [field][64]
@@ -70,7 +62,9 @@ enum {
 // wavefront evaluates at once, l its lane) keeps field f at
 // [(c * NFIELD + f) * 64 + l].
 // Reaction 32-bit fields, read for every reaction:
-//   RH_HDR  nf | nb << 2 | rev << 4 | kind << 6 | fot << 9 | GEN << 12
+//   RH_HDR  nf | nb << 2 | rev << 4 | kind << 6 | fot << 9 | GEN << 12 |
+//           SQ << 13 (bit i: order of reactant i is 2, bit 3 + i: of product i) |
+//           POW << 19 (some order is neither 1 nor 2)
 //   RH_IDX  fi0 | fi1 << 8 | fi2 << 16 | bi0 << 24;  RH_IDX2  bi1 | bi2 << 8
 //   RH_FNU.. RH_SUMS  stoichiometric coefficients, orders and their sum as
 //   float, exact for the small integers and halves of most mechanisms; a
@@ -78,7 +72,8 @@ enum {
 //   the double table instead.
 enum { RH_HDR, RH_IDX, RH_IDX2, RH_FNU, RH_BNU = RH_FNU + kWP, RH_FO = RH_BNU + kWP,
        RH_BO = RH_FO + kWP, RH_SUMS = RH_BO + kWP, RH_NFIELD };
-constexpr unsigned kRhGen = 1u << 12;
+constexpr unsigned kRhGen = 1u << 12, kRhPow = 1u << 19;
+constexpr int kRhSq = 13;
 // reaction double fields: the Arrhenius triple read for every reaction, then
 // what only some reactions read (fall-off, explicit reverse, GEN copies)
 enum {
@@ -119,6 +114,30 @@ struct WaveParams {
     WMech M;
     int exact_dkp;  // 1: exact d(Kp)/dT instead of the reference's sign convention
 };
+
+// The kernel's arguments, read again (scalar loads) wherever a phase of a
+// persistent kernel starts: kept live through the Newton loop they would
+// occupy more scalar registers than there are and be moved to and from vector
+// lanes instead.
+typedef const __attribute__((address_space(4))) WaveParams KWaveParams;
+__device__ __forceinline__ KWaveParams *wave_args() {
+    KWaveParams *k = (KWaveParams *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));  // a new value to the compiler: loads are not merged with earlier ones
+    return k;
+}
+__device__ __forceinline__ WMech wave_mech() {
+    KWaveParams *k = wave_args();
+    WMech M;
+    M.ns = k->M.ns;
+    M.nr = k->M.nr;
+    M.nrp = k->M.nrp;
+    M.sp = k->M.sp;
+    M.rh = k->M.rh;
+    M.rd = k->M.rd;
+    M.eff = k->M.eff;
+    M.efft = k->M.efft;
+    return M;
+}
 
 // Reads of the per-reaction tables through buffer resources: the lane is
 // the one vector offset, the chunk and field a scalar offset, so a table read
@@ -394,22 +413,20 @@ __device__ __forceinline__ void wreaction(const WMech &M, int ch, int lane, cons
     const int nf = hdr & 3u, nb = (hdr >> 2) & 3u, rev = (hdr >> 4) & 3u, kind = (hdr >> 6) & 7u;
     const int fi[kWP] = {(int)(ix & 255u), (int)((ix >> 8) & 255u), (int)((ix >> 16) & 255u)};
     const int bi[kWP] = {(int)(ix >> 24), (int)(ix2 & 255u), (int)((ix2 >> 8) & 255u)};
-    double fnu[kWP], bnu[kWP], fo[kWP], bo[kWP], cf[kWP], cb[kWP];
+    // everything a plain reaction needs is requested before the first use
+    double fnu[kWP], bnu[kWP], cf[kWP], cb[kWP];
+#pragma unroll
+    for (int i = 0; i < kWP; ++i) {
+        fnu[i] = ldf(tb, RH_FNU + i, ch, lane);
+        bnu[i] = ldf(tb, RH_BNU + i, ch, lane);
+    }
+    const double A = ldd(tb, RD_A, ch, lane), b = ldd(tb, RD_B, ch, lane),
+                 Ta = ldd(tb, RD_TA, ch, lane);
     if (hdr & kRhGen) {
 #pragma unroll
         for (int i = 0; i < kWP; ++i) {
             fnu[i] = ldd(tb, RD_FNU + i, ch, lane);
             bnu[i] = ldd(tb, RD_BNU + i, ch, lane);
-            fo[i] = ldd(tb, RD_FO + i, ch, lane);
-            bo[i] = ldd(tb, RD_BO + i, ch, lane);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < kWP; ++i) {
-            fnu[i] = ldf(tb, RH_FNU + i, ch, lane);
-            bnu[i] = ldf(tb, RH_BNU + i, ch, lane);
-            fo[i] = ldf(tb, RH_FO + i, ch, lane);
-            bo[i] = ldf(tb, RH_BO + i, ch, lane);
         }
     }
 #pragma unroll
@@ -417,12 +434,10 @@ __device__ __forceinline__ void wreaction(const WMech &M, int ch, int lane, cons
         cf[i] = i < nf ? sc[fi[i]] : 1.0;
         cb[i] = i < nb ? sc[bi[i]] : 1.0;
     }
-    const double A = ldd(tb, RD_A, ch, lane), b = ldd(tb, RD_B, ch, lane),
-                 Ta = ldd(tb, RD_TA, ch, lane);
     // third-body concentration, summed in species order (thirdBodyEfficiency::M)
     double Mtb = 0.0;
     if (kind != 0) {
-#pragma unroll 8
+#pragma unroll 16
         for (int k = 0; k < M.ns; ++k) Mtb += lde(tb, ch, lane, k) * sc[k];
     }
     double kf, k0 = 0.0, kinf = 0.0, Pr = 0.0, F = 1.0;
@@ -504,12 +519,39 @@ __device__ __forceinline__ void wreaction(const WMech &M, int ch, int lane, cons
         if (kind == 1) kr = Mtb * kr;
     }
     // concentration powers c^ord of every participant, computed once and
-    // reused by q, dq/dc and dq/dT (absent participants contribute 1)
-    double pf[kWP], pb[kWP];
+    // reused by q, dq/dc and dq/dT (absent participants contribute 1), and their
+    // derivatives: orders 1 and 2 by a select, others (kRhPow) in general
+    double pf[kWP], pb[kWP], df[kWP], db[kWP];
 #pragma unroll
     for (int i = 0; i < kWP; ++i) {
-        pf[i] = i < nf ? rpow(cf[i], fo[i]) : 1.0;
-        pb[i] = i < nb ? rpow(cb[i], bo[i]) : 1.0;
+        const bool f2 = hdr >> (kRhSq + i) & 1u, b2 = hdr >> (kRhSq + kWP + i) & 1u;
+        pf[i] = f2 ? cf[i] * cf[i] : cf[i];
+        pb[i] = b2 ? cb[i] * cb[i] : cb[i];
+        df[i] = f2 ? 2.0 * cf[i] : 1.0;
+        db[i] = b2 ? 2.0 * cb[i] : 1.0;
+    }
+    if (hdr & kRhPow) {
+        auto dpow = [](double c, double ord) {
+            if (ord == 1.0) return 1.0;
+            if (ord < 1.0) return c > kTiny ? ord * pow_ool(c, ord - 1.0) : 0.0;
+            return ord * rpow(c, ord - 1.0);
+        };
+        for (int i = 0; i < kWP; ++i) {
+            const double fo = (hdr & kRhGen) ? ldd(tb, RD_FO + i, ch, lane) : ldf(tb, RH_FO + i, ch, lane);
+            const double bo = (hdr & kRhGen) ? ldd(tb, RD_BO + i, ch, lane) : ldf(tb, RH_BO + i, ch, lane);
+            const double c = i == 0 ? cf[0] : i == 1 ? cf[1] : cf[2];
+            const double d = i == 0 ? cb[0] : i == 1 ? cb[1] : cb[2];
+            const double p = i < nf ? rpow(c, fo) : 1.0, q = i < nb ? rpow(d, bo) : 1.0;
+            const double dp = i < nf ? dpow(c, fo) : 1.0, dq = i < nb ? dpow(d, bo) : 1.0;
+#pragma unroll
+            for (int k = 0; k < kWP; ++k)
+                if (k == i) {
+                    pf[k] = p;
+                    pb[k] = q;
+                    df[k] = dp;
+                    db[k] = dq;
+                }
+        }
     }
     const double prf = pf[0] * pf[1] * pf[2], prb = pb[0] * pb[1] * pb[2];
     const double qf = kf * prf, qr = kr * prb;
@@ -530,14 +572,9 @@ __device__ __forceinline__ void wreaction(const WMech &M, int ch, int lane, cons
     // participants' powers
 #pragma unroll
     for (int i = 0; i < kWP; ++i) {
-        auto dpow = [](double c, double ord) {
-            if (ord == 1.0) return 1.0;
-            if (ord < 1.0) return c > kTiny ? ord * pow_ool(c, ord - 1.0) : 0.0;
-            return ord * rpow(c, ord - 1.0);
-        };
         const int i1 = (i + 1) % kWP, i2 = (i + 2) % kWP;
-        o.dqf[i] = i < nf ? kf * dpow(cf[i], fo[i]) * (pf[i1] * pf[i2]) : 0.0;
-        o.dqr[i] = i < nb ? kr * dpow(cb[i], bo[i]) * (pb[i1] * pb[i2]) : 0.0;
+        o.dqf[i] = i < nf ? kf * df[i] * (pf[i1] * pf[i2]) : 0.0;
+        o.dqr[i] = i < nb ? kr * db[i] * (pb[i1] * pb[i2]) : 0.0;
     }
     // third-body / fall-off terms q dln(gamma)/dc_j = gam * eff_j
     double gam = 0.0;
@@ -594,12 +631,6 @@ struct WaveLDS {
     double c[N], G[N], dG[N], H[N];  // species k in [k]
     double Cp[kCpLds ? N : 1], dCp[kCpLds ? N : 1];
     double w[N];      // net production rates omega_k
-#if OHC_LU_BCAST == 0
-    // pivot row of the current elimination step (element j at [2 j], b at
-    // [2 N]): the stride keeps the writes single 64-bit stores straight from
-    // the row's registers instead of packed 128-bit stores that need copies
-    double prow[2 * N + 1];
-#endif
 };
 
 // dy/dt (and the Jacobian into L.J when WITH_J) at the wavefront-distributed
@@ -683,22 +714,34 @@ __device__ __forceinline__ double wave_eval(const WMech &M, WaveLDS<N> &L, doubl
             }
             const RxnTab tb = rxn_tab(M);
             while (tbm) {
-                const int sl = __ffsll((long long)tbm) - 1;
-                tbm &= tbm - 1ull;
-                const double e = lde_col(tb, base + sl, lane);  // eff_rj, zero past ns
-                const int nf = __builtin_amdgcn_readlane(o.nf, sl),
-                          nb = __builtin_amdgcn_readlane(o.nb, sl);
+                // up to four reactions' efficiencies eff_rj (zero past ns) are
+                // requested together
+                int sl[4], cnt = 0;
+                double e[4];
 #pragma unroll
-                for (int i = 0; i < kWP; ++i) {
-                    if (i < nf) {
-                        const int k = __builtin_amdgcn_readlane(o.fi[i], sl);
-                        const double v = rdlane(o.fnu[i], sl) * e;
-                        if (lane < ns) lds_add(&L.J[k * WaveLDS<N>::JS + lane], v);
-                    }
-                    if (i < nb) {
-                        const int k = __builtin_amdgcn_readlane(o.bi[i], sl);
-                        const double v = rdlane(o.bnu[i], sl) * e;
-                        if (lane < ns) lds_add(&L.J[k * WaveLDS<N>::JS + lane], v);
+                for (int q = 0; q < 4; ++q) {
+                    sl[q] = tbm ? __builtin_ctzll(tbm) : sl[0];
+                    cnt += tbm ? 1 : 0;
+                    tbm &= tbm - 1ull;
+                    e[q] = lde_col(tb, base + sl[q], lane);
+                }
+                for (int q = 0; q < cnt; ++q) {
+                    const int s1 = q == 0 ? sl[0] : q == 1 ? sl[1] : q == 2 ? sl[2] : sl[3];
+                    const double eq = q == 0 ? e[0] : q == 1 ? e[1] : q == 2 ? e[2] : e[3];
+                    const int nf = __builtin_amdgcn_readlane(o.nf, s1),
+                              nb = __builtin_amdgcn_readlane(o.nb, s1);
+#pragma unroll
+                    for (int i = 0; i < kWP; ++i) {
+                        if (i < nf) {
+                            const int k = __builtin_amdgcn_readlane(o.fi[i], s1);
+                            const double v = rdlane(o.fnu[i], s1) * eq;
+                            if (lane < ns) lds_add(&L.J[k * WaveLDS<N>::JS + lane], v);
+                        }
+                        if (i < nb) {
+                            const int k = __builtin_amdgcn_readlane(o.bi[i], s1);
+                            const double v = rdlane(o.bnu[i], s1) * eq;
+                            if (lane < ns) lds_add(&L.J[k * WaveLDS<N>::JS + lane], v);
+                        }
                     }
                 }
             }
@@ -746,21 +789,28 @@ __device__ __forceinline__ double wave_eval(const WMech &M, WaveLDS<N> &L, doubl
     return sp ? w : (lane == ns ? -dT : 0.0);
 }
 
-// Solve (diag I - h J) x = b with the Jacobian rows in LDS: lane i owns row i;
-// partial pivoting as SquareMatrix::LUDecomposeDPivoting (largest |pivot| to
-// 2^-20 relative, lowest row among those), forward substitution folded into the
-// elimination.  Returns x_i in lane i.  The elimination steps are unrolled at
-// compile time, so step k touches only the N - k - 1 columns right of the
-// pivot; FULL (n == N) drops the per-step bounds, so that the whole
-// factorisation is one straight-line block the compiler can schedule across
-// steps.  The pivot row reaches the other lanes as OHC_LU_BCAST selects; each
-// pivot row keeps its step and reciprocal in two registers for the back
-// substitution.
+// a_j <- a_j - l a_pj for the columns j = K .. N-1.  The pivot row's elements
+// are read eight at a time ahead of their multiply-adds: an SGPR written by
+// v_readlane may be read by the next vector instruction only after two wait
+// states, which the compiler's order (two reads, the wait, the multiply-add)
+// pays for every element.
+template <int K, int N>
+__device__ __forceinline__ void wave_lu_update(double (&a)[N], double l, int p) {
+    sfor<0, (N - K + 7) / 8>([&](auto bc) {
+        constexpr int j0 = K + 8 * bc, j1 = j0 + 8 < N ? j0 + 8 : N;
+        double t[8];
+        sfor<j0, j1>([&](auto j) { t[j - j0] = rdlane(a[j], p); });
+        __builtin_amdgcn_sched_barrier(0);
+        sfor<j0, j1>([&](auto j) { a[j] = fma(-l, t[j - j0], a[j]); });
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+
+// Row i of diag I - h J into lane i's registers.
 template <int N, bool FULL>
-__device__ __forceinline__ double wave_lu_solve_n(WaveLDS<N> &L, int n, double h, double b,
-                                                  double diag) {
+__device__ __forceinline__ void wave_lu_rows(const WaveLDS<N> &L, int n, double h, double diag,
+                                             double (&a)[N]) {
     const int lane = threadIdx.x;
-    if (FULL) n = N;
     const bool act = lane < n;
     // every lane loads a row that exists (lanes past the system read row 0),
     // so the N loads issue back to back without a branch and a wait each.
@@ -768,7 +818,6 @@ __device__ __forceinline__ double wave_lu_solve_n(WaveLDS<N> &L, int n, double h
     // never pivots, so no other lane reads them, and their b and x are not
     // used.
     const double *Jr = L.J + (act ? lane : 0) * WaveLDS<N>::JS;
-    double a[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         // -h J, then + diag on the diagonal: two roundings, as the reference
@@ -779,6 +828,84 @@ __device__ __forceinline__ double wave_lu_solve_n(WaveLDS<N> &L, int n, double h
         const bool dj = __builtin_amdgcn_inverse_ballot_w64(1ull << j);  // lane == j
         a[j] = ((FULL || act) && dj) ? v + diag : v;
     }
+}
+
+// The solve of wave_lu_solve_n with the pivot rows of an earlier factorisation
+// (lane k of perm: the row of step k).  The order of pivots seldom changes
+// from one Newton iteration to the next, so instead of searching each column
+// (a chain of six lane exchanges, a scalar read and a ballot per step) every step only
+// checks that the expected row is the one the search would pick -- no unused
+// row exceeds the high word of its |a_ik|, no lower one equals it -- and
+// collects the failures in one mask.  The arithmetic is that of the search's path, so a solve
+// that returns true has its bits; one that returns false (an unexpected pivot,
+// or a NaN anywhere in the solution) is to be repeated with the search.
+template <int N, bool FULL>
+__device__ __forceinline__ bool wave_lu_expected(const WaveLDS<N> &L, int n, double h, double b,
+                                                 double diag, int perm, double &xout) {
+    if (FULL) n = N;
+    double a[N];
+    wave_lu_rows<N, FULL>(L, n, h, diag, a);
+    unsigned long long avail = FULL && N < 64 ? (1ull << (N & 63)) - 1ull
+                                              : __builtin_amdgcn_ballot_w64((int)threadIdx.x < n);
+    unsigned long long off = 0ull;  // rows that break the expectation
+    double rpv = 0.0;
+    sfor<0, N>([&](auto kc) {
+        constexpr int k = kc;
+        if (FULL || k < n) {
+            const int p = __builtin_amdgcn_readlane(perm, k);
+            const unsigned hi = (unsigned)__double2hiint(a[k]) & 0x7fffffffu;
+            const unsigned hp = (unsigned)__builtin_amdgcn_readlane((int)hi, p);
+            const unsigned long long pm = 1ull << p;
+            off |= (avail & (__builtin_amdgcn_ballot_w64(hi > hp) |
+                             (__builtin_amdgcn_ballot_w64(hi == hp) & (pm - 1ull)))) |
+                   (pm & ~avail);
+            const double pk = rdlane(a[k], p);
+            // frcp without its zero and infinity cases: those come out NaN here
+            double rp = __builtin_amdgcn_rcp(pk);
+            rp = fma(fma(-pk, rp, 1.0), rp, rp);
+            rp = fma(fma(-pk, rp, 1.0), rp, rp);
+            rpv = __builtin_amdgcn_inverse_ballot_w64(pm) ? rp : rpv;
+            avail &= ~pm;
+            const double l = __builtin_amdgcn_inverse_ballot_w64(avail) ? a[k] * rp : 0.0;
+            wave_lu_update<k + 1>(a, l, p);
+            b = fma(-l, rdlane(b, p), b);
+        }
+    });
+    double x = 0.0;
+    sfor<0, N>([&](auto kk) {
+        constexpr int k = N - 1 - kk;
+        if (FULL || k < n) {
+            const int p = __builtin_amdgcn_readlane(perm, k);
+            const double t = b * rpv, xk = rdlane(t, p);
+            b = fma(-a[k], xk, b);
+            x = __builtin_amdgcn_inverse_ballot_w64(1ull << p) ? t : x;
+        }
+    });
+    // lane k takes x_k from the row of step k; lanes past the system hold 0
+    const double v = bperm(x, perm * 4);
+    xout = (int)threadIdx.x < n ? v : 0.0;
+    return off == 0ull && !__any(isnan(x));
+}
+
+// Solve (diag I - h J) x = b with the Jacobian rows in LDS: lane i owns row i;
+// partial pivoting as SquareMatrix::LUDecomposeDPivoting (largest |pivot| to
+// 2^-20 relative, lowest row among those), forward substitution folded into the
+// elimination.  Returns x_i in lane i and the pivot row of step k in lane k of
+// perm.  The elimination steps are unrolled at compile time, so step k touches
+// only the N - k - 1 columns right of the pivot; FULL (n == N) drops the
+// per-step bounds, so that the whole factorisation is one straight-line block
+// the compiler can schedule across steps.  The pivot row reaches the other
+// lanes by v_readlane pairs (through LDS or ds_bpermute it was slower); each
+// pivot row keeps its step and reciprocal in two registers for the back
+// substitution.
+template <int N, bool FULL>
+__device__ __forceinline__ double wave_lu_solve_n(WaveLDS<N> &L, int n, double h, double b,
+                                                  double diag, int &perm) {
+    const int lane = threadIdx.x;
+    if (FULL) n = N;
+    const bool act = lane < n;
+    double a[N];
+    wave_lu_rows<N, FULL>(L, n, h, diag, a);
     // rows not yet used as a pivot, as a lane mask: the per-row predicates
     // of an elimination step are scalar mask operations
     unsigned long long avail = __builtin_amdgcn_ballot_w64(act);
@@ -819,25 +946,8 @@ __device__ __forceinline__ double wave_lu_solve_n(WaveLDS<N> &L, int n, double h
             const double l = __builtin_amdgcn_inverse_ballot_w64(avail) ? a[k] * rp : 0.0;
             // columns j >= n hold zeros in every row and stay zero, so the
             // update needs no per-column predicate
-#if OHC_LU_BCAST == 2
-            const int p4 = p * 4;
-            sfor<k + 1, N>([&](auto j) { a[j] = fma(-l, bperm(a[j], p4), a[j]); });
-            b = fma(-l, bperm(b, p4), b);
-#elif OHC_LU_BCAST == 1
-            sfor<k + 1, N>([&](auto j) { a[j] = fma(-l, rdlane(a[j], p), a[j]); });
+            wave_lu_update<k + 1>(a, l, p);
             b = fma(-l, rdlane(b, p), b);
-#else
-            if (__builtin_amdgcn_inverse_ballot_w64(pm)) {
-                sfor<k + 1, N>([&](auto j) { L.prow[2 * j] = a[j]; });
-                L.prow[2 * N] = b;
-            }
-            // (the block is one wavefront, whose LDS accesses complete in
-            // program order: the reads below see the row, and the next
-            // step's row cannot overwrite them)
-            __builtin_amdgcn_wave_barrier();
-            sfor<k + 1, N>([&](auto j) { a[j] = fma(-l, L.prow[2 * j], a[j]); });
-            b = fma(-l, L.prow[2 * N], b);
-#endif
         }
     });
     double xo = 0.0;  // the unknown of this row's step, set at that step
@@ -862,6 +972,7 @@ __device__ __forceinline__ double wave_lu_solve_n(WaveLDS<N> &L, int n, double h
     const int dst = (stepv < n ? stepv : lane) * 4;
     const int lo = __builtin_amdgcn_ds_permute(dst, __double2loint(xo));
     const int hi = __builtin_amdgcn_ds_permute(dst, __double2hiint(xo));
+    perm = __builtin_amdgcn_ds_permute(dst, lane);
     // a column whose remaining rows are all NaN leaves steps without a
     // pivot row: the solution is NaN, as the reference's division by a NaN
     // pivot makes it (the caller then rejects the Newton step)
@@ -869,9 +980,24 @@ __device__ __forceinline__ double wave_lu_solve_n(WaveLDS<N> &L, int n, double h
 }
 template <int N>
 __device__ __forceinline__ double wave_lu_solve(WaveLDS<N> &L, int n, double h, double b,
-                                                double diag = 1.0) {
-    return n == N ? wave_lu_solve_n<N, true>(L, n, h, b, diag)
-                  : wave_lu_solve_n<N, false>(L, n, h, b, diag);
+                                                double diag, int &perm) {
+    return n == N ? wave_lu_solve_n<N, true>(L, n, h, b, diag, perm)
+                  : wave_lu_solve_n<N, false>(L, n, h, b, diag, perm);
+}
+// The same solve, first with the pivot rows of the wavefront's last
+// factorisation (perm; any values to begin with), where that pays: on the
+// 54-species mechanism 3 % of the factorisations have to be repeated (49,152
+// cells: 438 -> 404 ms together with the batched reads of wave_lu_update), on
+// the 32-species one 23 %, which costs what the checks save.
+template <int N>
+__device__ __forceinline__ double wave_lu_solve_next(WaveLDS<N> &L, int n, double h, double b,
+                                                     double diag, int &perm) {
+    if constexpr (N <= 40) return wave_lu_solve<N>(L, n, h, b, diag, perm);
+    double x;
+    const bool ok = n == N ? wave_lu_expected<N, true>(L, n, h, b, diag, perm, x)
+                           : wave_lu_expected<N, false>(L, n, h, b, diag, perm, x);
+    if (!ok) x = wave_lu_solve_n<N, false>(L, n, h, b, diag, perm);
+    return x;
 }
 
 // Persistent integrator: each wavefront takes one cell at a time from the
@@ -892,39 +1018,40 @@ __device__ __forceinline__ double wave_lu_solve(WaveLDS<N> &L, int n, double h, 
 // Jacobian, LU, error norms and sums), ImplicitEuler only.
 template <int N, int FLOW, int METH = 0, class F = double>
 __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const WaveParams WP) {
-    const LaneParams &P = WP.L;
-    const WMech &M = WP.M;
-    const int lane = threadIdx.x, ns = M.ns, n = ns + 1;
+    KWaveParams *kp = wave_args();
+    const int lane = threadIdx.x, ns = kp->M.ns, n = ns + 1;
     __shared__ WaveLDS<N> L;
     __shared__ unsigned long long s_cell;
     const bool sp = lane < ns;
-    const double W = sp ? M.sp[SP_W * 64 + lane] : 1.0;
-    const double errg = pow(P.maxsc / P.safe, -1.0 / P.alpha);
+    const double W = sp ? kp->M.sp[SP_W * 64 + lane] : 1.0;
+    int perm = lane;  // pivot rows of the last factorisation
+    const double errg = pow(kp->L.maxsc / kp->L.safe, -1.0 / kp->L.alpha);
     long long c_cells = 0, c_steps = 0, c_att = 0, c_newt = 0, c_rhs = 0, c_maxs = 0, c_fail = 0;
     double dtmin = __builtin_huge_val();
     for (;;) {
-        if (lane == 0) s_cell = atomicAdd(P.counter, 1ull);
+        kp = wave_args();
+        if (lane == 0) s_cell = atomicAdd(kp->L.counter, 1ull);
         __syncthreads();
         const unsigned long long qi = s_cell;
         __syncthreads();
-        if (qi >= (unsigned long long)P.n) break;
-        const long long cell = P.order ? (long long)P.order[qi] : (long long)qi;
-        const double T0 = P.T[cell];
-        const double dtc = P.dt[cell] * P.dtFactor;
-        const double sub_in = P.subDt[cell];
-        if (T0 < P.Tthr) {
+        if (qi >= (unsigned long long)kp->L.n) break;
+        const long long cell = kp->L.order ? (long long)kp->L.order[qi] : (long long)qi;
+        const double T0 = kp->L.T[cell];
+        const double dtc = kp->L.dt[cell] * kp->L.dtFactor;
+        const double sub_in = kp->L.subDt[cell];
+        if (T0 < kp->L.Tthr) {
             if (lane == 0) {
-                P.subDt[cell] = dtc;
-                if (P.cost) P.cost[cell] = 0;
+                kp->L.subDt[cell] = dtc;
+                if (kp->L.cost) kp->L.cost[cell] = 0;
             }
-            if (P.mode == 0 && sp) P.R[lane * P.ldR + cell] = 0.0;
+            if (kp->L.mode == 0 && sp) kp->L.R[lane * kp->L.ldR + cell] = 0.0;
             continue;
         }
-        const double rho = P.rho[cell];
-        const double pr = FLOW == 0 ? P.p[cell] : rho;
-        const double c0 = sp ? rho * P.Y[lane * P.ldY + cell] / W : 0.0;
+        const double rho = kp->L.rho[cell];
+        const double pr = FLOW == 0 ? kp->L.p[cell] : rho;
+        const double c0 = sp ? rho * kp->L.Y[lane * kp->L.ldY + cell] / W : 0.0;
         double y = sp ? c0 : (lane == ns ? T0 : 0.0);  // chemistry state, lane i = y_i
-        double subDt = fmin(dtc, fmin(sub_in > 0.0 ? sub_in : dtc, P.dt_max));
+        double subDt = fmin(dtc, fmin(sub_in > 0.0 ? sub_in : dtc, kp->L.dt_max));
         double left = dtc;
         long long csteps = 0, citer = 0;
         bool failed = false;
@@ -940,7 +1067,7 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
             bool last = false, done = false;
             double yl1 = y, lts0 = 0.0, lts1 = 0.0, lts2 = 0.0;
             double h0 = y, h1 = y, h2 = y;  // BDF23 step-start history (yklast_)
-            for (int nstep = 0; nstep < P.max_steps; ++nstep) {
+            for (int nstep = 0; nstep < kp->L.max_steps; ++nstep) {
                 const double y0 = y;
                 int order = 0;
                 if constexpr (METH == 3) {
@@ -981,7 +1108,7 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                         f0 = fnext;
                     } else {
                         ++c_rhs;
-                        f0 = wave_eval<N, FLOW, false>(M, L, y0, WP.exact_dkp);
+                        f0 = wave_eval<N, FLOW, false>(wave_mech(), L, y0, wave_args()->exact_dkp);
                     }
                     fnext_ok = false;
                 }
@@ -1011,7 +1138,7 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                     double lastErr = 0.0, maxErr = 0.0;
                     bool conv = true;
                     for (;;) {
-                        const double f = wave_eval<N, FLOW, true, F>(M, L, yk, WP.exact_dkp);
+                        const double f = wave_eval<N, FLOW, true, F>(wave_mech(), L, yk, wave_args()->exact_dkp);
                         ++c_newt;
                         ++citer;
                         const double h = METH == 2 ? 0.5 * dtl : dtl;
@@ -1024,14 +1151,16 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                         } else {
                             rhs = -yk + y0 + dtl * f;
                         }
-                        const double d = wave_lu_solve<N>(L, n, h, lane < n ? rhs : 0.0, dg);
+                        const double d =
+                            wave_lu_solve_next<N>(L, n, h, lane < n ? rhs : 0.0, dg, perm);
+                        kp = wave_args();
                         if (__any(lane < n && bad(d))) {
                             conv = false;
                             maxErr = 1000.0;
                             break;
                         }
                         yk += d;
-                        const double tol = P.atol + P.rtol * fabs(yk);
+                        const double tol = kp->L.atol + kp->L.rtol * fabs(yk);
                         maxErr = wmax(lane < n ? fabs(d) * frcp(tol) : 0.0);
                         if (count > 0 && (maxErr / fmax(lastErr, kTiny)) > 2 && count > 5) {
                             conv = false;
@@ -1050,7 +1179,7 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                             break;
                         }
                         if (maxErr <= 1.0) break;
-                        if (citer > P.max_cell_iters) {
+                        if (citer > kp->L.max_cell_iters) {
                             conv = false;
                             failed = true;
                             break;
@@ -1065,7 +1194,7 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                         if constexpr (METH == 3) {
                             if (nstep <= 2) {
                                 ++c_rhs;
-                                const double f = wave_eval<N, FLOW, false>(M, L, yk, WP.exact_dkp);
+                                const double f = wave_eval<N, FLOW, false>(wave_mech(), L, yk, wave_args()->exact_dkp);
                                 e = yk - y0 - dtl * f;
                             } else {
                                 const double D = lts0, D1 = lts1, D2 = lts2;
@@ -1075,7 +1204,7 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                             }
                         } else if constexpr (METH == 2) {
                             ++c_rhs;
-                            fk = wave_eval<N, FLOW, false>(M, L, yk, WP.exact_dkp);
+                            fk = wave_eval<N, FLOW, false>(wave_mech(), L, yk, wave_args()->exact_dkp);
                             if (nstep == 0) {
                                 e = yk - y0 - dtl * fk;
                             } else {
@@ -1087,7 +1216,7 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                             }
                         } else if (nstep == 0) {
                             ++c_rhs;
-                            const double f = wave_eval<N, FLOW, false, F>(M, L, yk, WP.exact_dkp);
+                            const double f = wave_eval<N, FLOW, false, F>(wave_mech(), L, yk, wave_args()->exact_dkp);
                             e = yk - y0 - dtl * f;
                         } else {
                             const double dtn = lts0, dtn1 = lts1;
@@ -1097,14 +1226,14 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                             e = (f1 * (yk - y0) - f2 * (y0 - yl1)) * LTEF;
                         }
                         const bool nan_y = __any(lane < n && isnan(yk));
-                        const double tol = P.atol_inc + P.rtol_inc * fmax(fabs(y0), fabs(yk));
+                        const double tol = kp->L.atol_inc + kp->L.rtol_inc * fmax(fabs(y0), fabs(yk));
                         const double m = wmax(lane < n ? fabs(e) * frcp(tol) : 0.0);
                         error = nan_y ? 1.5 : m;
                     }
                     // checkNewY, then the step-size control of adaptiveSolve
                     const double y0T = rdlane(y0, ns), ykT = rdlane(yk, ns);
-                    const bool ok = !((ykT - y0T) > P.Talpha * y0T);
-                    if (!ok) dtl *= P.Tbeta;
+                    const bool ok = !((ykT - y0T) > kp->L.Talpha * y0T);
+                    if (!ok) dtl *= kp->L.Tbeta;
                     if (!ok && chk < 100) {
                         ++chk;
                         if (dtl <= kVeryTiny) {
@@ -1117,7 +1246,7 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                         if (lastError < error && error < 5.0) break;
                     }
                     if (error > 1.0) {
-                        dtl *= fmax(P.safe * pow(error, -P.alpha), P.minsc);
+                        dtl *= fmax(kp->L.safe * pow(error, -kp->L.alpha), kp->L.minsc);
                         if (dtl <= kVeryTiny) {
                             failed = true;
                             break;
@@ -1140,9 +1269,9 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
                     fnext_ok = last_conv;
                 }
                 if (error > errg)
-                    dt = fmin(fmax(P.safe * pow(error, -P.alpha), P.minsc), P.maxsc) * dtl;
+                    dt = fmin(fmax(kp->L.safe * pow(error, -kp->L.alpha), kp->L.minsc), kp->L.maxsc) * dtl;
                 else
-                    dt = fmax(P.safe * P.maxsc * dtl, dtl);
+                    dt = fmax(kp->L.safe * kp->L.maxsc * dtl, dtl);
                 ++c_steps;
                 ++csteps;
                 if ((t - tn) * tn >= 0) {
@@ -1155,14 +1284,15 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
             if (!done) tn = t;  // step budget exhausted: time reached
             left -= tn;
         }
+        kp = wave_args();
         if (failed) ++c_fail;
         // outputs (chemistrySource.cpp:1494-1609)
         if (lane == 0) {
-            P.subDt[cell] = subDt;
-            if (P.cost) P.cost[cell] = (int)(citer < 0x7fffffffll ? citer : 0x7fffffffll);
+            kp->L.subDt[cell] = subDt;
+            if (kp->L.cost) kp->L.cost[cell] = (int)(citer < 0x7fffffffll ? citer : 0x7fffffffll);
         }
-        if (P.mode == 0) {
-            if (sp) P.R[lane * P.ldR + cell] = (y - c0) * (1.0 / dtc) * W;
+        if (kp->L.mode == 0) {
+            if (sp) kp->L.R[lane * kp->L.ldR + cell] = (y - c0) * (1.0 / dtc) * W;
         } else {
             // ciToYi (chemistrySource.cpp:1222-1240)
             const double yy = sp ? fmax(0.0, y) : 0.0;
@@ -1171,24 +1301,24 @@ __global__ __launch_bounds__(64, (N <= 40 ? 3 : 2)) void ie_wave_kernel(const Wa
             const double yv = yy * W * rr;
             const double ys = wsum(yv);
             const double ri = 1.0 / ys;
-            if (sp) P.Yout[lane * P.ldY + cell] = ys != 1.0 ? yv * ri : yv;
+            if (sp) kp->L.Yout[lane * kp->L.ldY + cell] = ys != 1.0 ? yv * ri : yv;
             const double Tn = rdlane(y, ns);
-            if (lane == 0) P.Tout[cell] = Tn;
+            if (lane == 0) kp->L.Tout[cell] = Tn;
         }
         ++c_cells;
         dtmin = fmin(dtmin, subDt);
         c_maxs = csteps > c_maxs ? csteps : c_maxs;
     }
     if (lane == 0) {
-        atomicAdd(&P.stats[0], (unsigned long long)c_cells);
-        atomicAdd(&P.stats[1], (unsigned long long)c_steps);
-        atomicAdd(&P.stats[2], (unsigned long long)c_att);
-        atomicAdd(&P.stats[3], (unsigned long long)c_newt);
-        atomicAdd(&P.stats[4], (unsigned long long)c_rhs);
-        atomicMax(&P.stats[5], (unsigned long long)c_maxs);
+        atomicAdd(&kp->L.stats[0], (unsigned long long)c_cells);
+        atomicAdd(&kp->L.stats[1], (unsigned long long)c_steps);
+        atomicAdd(&kp->L.stats[2], (unsigned long long)c_att);
+        atomicAdd(&kp->L.stats[3], (unsigned long long)c_newt);
+        atomicAdd(&kp->L.stats[4], (unsigned long long)c_rhs);
+        atomicMax(&kp->L.stats[5], (unsigned long long)c_maxs);
         if (dtmin < __builtin_huge_val())
-            atomicMin(&P.stats[6], (unsigned long long)__double_as_longlong(dtmin));
-        atomicAdd(&P.stats[7], (unsigned long long)c_fail);
+            atomicMin(&kp->L.stats[6], (unsigned long long)__double_as_longlong(dtmin));
+        atomicAdd(&kp->L.stats[7], (unsigned long long)c_fail);
     }
 }
 
@@ -1415,7 +1545,8 @@ __global__ __launch_bounds__(64) void lu_wave_kernel(const LuParams P) {
         L.J[(e / n) * WaveLDS<N>::JS + e % n] = P.A[(int64_t)e * P.ldA + m];
     __syncthreads();
     const double b = lane < n ? P.b[(int64_t)lane * P.ldb + m] : 0.0;
-    const double x = wave_lu_solve<N>(L, n, -1.0, b, 0.0);
+    int perm = 0;
+    const double x = wave_lu_solve<N>(L, n, -1.0, b, 0.0, perm);
     if (lane < n) P.x[(int64_t)lane * P.ldx + m] = x;
 }
 
