@@ -92,7 +92,8 @@ def build(verbose: bool = True) -> Path:
     # Horner chains whose lowest coefficient is 0; without signed zeros those
     # adds fold away (only the sign of an exact zero result can change).
     jobs = [(src, BUILD / (src.stem + ".hip.o"), ["-fno-signed-zeros"] if src == reg else [])
-            for src in [CSRC / "ohc_api.cpp", reg, CSRC / "wave_dispatch.hip", CSRC / "props_table.hip",
+            for src in [CSRC / "ohc_api.cpp", reg, CSRC / "wave_dispatch.hip",
+                        CSRC / "props_table.hip", CSRC / "source_table.hip",
                         CSRC / "surrogate_api.hip", CSRC / "sched.hip", CSRC / "noalloc.hip"]]
     jobs += [(CSRC / "wave_size.hip", BUILD / f"wave_{n}.hip.o", [f"-DOHC_WAVE_N={n}"])
              for n in WAVE_SIZES]

@@ -31,6 +31,8 @@ struct ohc_ctx {
     ohcd::WMech wm{};           // device tables of the generic kernels
     void *d_wm = nullptr;       // one allocation holding them
     ohcd::PairTab pair{};       // pair constants of the mixture rules (in d_wm)
+    ohcd::SrcTab src{};         // reaction records of the source terms (in d_wm; null: the
+                                // mechanism needs the general kernel)
     int grid = 0;  // persistent integrator grid (single-wavefront blocks)
     int cus = 0;         // compute units of the device
     int max_per_cu = 0;  // resident integrator blocks per CU the kernel allows
@@ -43,6 +45,8 @@ struct ohc_ctx {
     int *d_cost = nullptr, *d_order = nullptr;
     unsigned *d_bins = nullptr;  // counting-sort buckets (2 * ohcs::kBins)
     bool in_slices = false;  // inside a sliced host-pointer call (one slice at a time)
+    int64_t sliced_n = 0;    // and the cells of the whole call: a choice of kernel by the number
+                             // of cells is the same for every slice
     std::string err, kname;
 };
 

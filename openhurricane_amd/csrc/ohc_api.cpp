@@ -71,9 +71,11 @@ bool host_slices(ohc_ctx *c, int64_t n, size_t bytes_per_cell, int64_t *m) {
 template <class F>
 int run_slices(ohc_ctx *c, int64_t n, int64_t m, F &&f) {
     c->in_slices = true;
+    c->sliced_n = n;
     int rc = OHC_OK;
     for (int64_t s = 0; s < n && rc == OHC_OK; s += m) rc = f(s, std::min(m, n - s));
     c->in_slices = false;
+    c->sliced_n = 0;
     return rc;
 }
 
@@ -254,12 +256,56 @@ int build_wmech(ohc_ctx *c) {
                 efft[((size_t)(q / 64) * 64 + k) * 64 + q % 64] = m.eff[(size_t)r * ns + k];
             }
     }
+    std::vector<double> rec((size_t)std::max(nr, 1) * SrcTab::kRec, 0.0);
+    bool rec_ok = c->wm.uniform_range && ns <= 56 && nr > 0;
+    c->src.first_tb = 0;
+    static_assert(SrcTab::kSum < SrcTab::kWords && SrcTab::kNasa + 14 <= SrcTab::kRec, "record");
+    for (int q = 0; q < nr; ++q) {
+        const int r = perm[q];
+        double *d = &rec[(size_t)q * SrcTab::kRec];
+        uint32_t u[SrcTab::kWords] = {}, hdr = rh[xh(RH_HDR, q)], last = 7u;
+        if (hdr & kRhGen) rec_ok = false;
+        if (m.kind[r] == OHC_RATE_ARRHENIUS) c->src.first_tb = q + 1;
+        int id[2 * kWP];
+        for (int p = 0; p < 2 * kWP; ++p) {
+            const int i = p % kWP;
+            const bool f = p < kWP, on = i < (f ? m.nf[r] : m.nb[r]);
+            id[p] = !on ? ns : f ? m.f_idx[r * P + i] : m.b_idx[r * P + i];
+            u[SrcTab::kRow + p / 2] |= (uint32_t)(id[p] * 64) << (16 * (p & 1));
+            u[SrcTab::kNu + p] = !on ? 0u : f ? fbits(-m.f_nu[r * P + i]) : fbits(m.b_nu[r * P + i]);
+            u[SrcTab::kOrd + p] = !on ? fbits(1.0) : fbits(f ? m.f_ord[r * P + i] : m.b_ord[r * P + i]);
+            if (on && i == 2) hdr |= SrcTab::kThree;
+            if (on && id[p] == ns - 1) last = (uint32_t)p;
+            if (on && m.kind[r] != OHC_RATE_ARRHENIUS)
+                d[SrcTab::kEff + p] = m.eff[(size_t)r * ns + id[p]];
+            for (int j = 0; j < p; ++j)
+                if (on && id[j] == id[p]) hdr |= SrcTab::kBoth;
+        }
+        u[SrcTab::kHdr] = hdr | last << SrcTab::kLast;
+        u[SrcTab::kSum] = rh[xh(RH_SUMS, q)];
+        std::memcpy(d, u, sizeof(u));
+        for (int i = 0; i < 3; ++i) {
+            d[SrcTab::kArr + i] = m.arr[3 * r + i];
+            d[SrcTab::kLow + i] = m.arr_lo[3 * r + i];
+            d[SrcTab::kRev + i] = m.arr_rev[3 * r + i];
+        }
+        for (int i = 0; i < 5; ++i) d[SrcTab::kFop + i] = m.fo[5 * r + i];
+        for (int side = 0; side < 2; ++side)
+            for (int i = 0; i < 7; ++i) {
+                double a = 0.0;
+                const int o = ((side == 0 ? SP_ALO : SP_AHI) + i) * 64;
+                auto add = [&](int k, double nu) { a += nu * sp[SP_W * 64 + k] * sp[o + k]; };
+                for (int j = 0; j < m.nf[r]; ++j) add(m.f_idx[r * P + j], -m.f_nu[r * P + j]);
+                for (int j = 0; j < m.nb[r]; ++j) add(m.b_idx[r * P + j], m.b_nu[r * P + j]);
+                d[SrcTab::kNasa + 7 * side + i] = a;
+            }
+    }
     // one device allocation, 256-byte aligned pieces
     auto al = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t b_sp = al(sp.size() * 8), b_rh = al(rh.size() * 4), b_rd = al(rd.size() * 8),
                  b_ef = al(eff.size() * 8), b_et = al(efft.size() * 8),
-                 b_pr = al(pair.size() * 8);
-    const size_t total = b_sp + b_rh + b_rd + b_ef + b_et + b_pr;
+                 b_pr = al(pair.size() * 8), b_rc = al(rec.size() * 8);
+    const size_t total = b_sp + b_rh + b_rd + b_ef + b_et + b_pr + b_rc;
     std::vector<unsigned char> h(total, 0);
     size_t off = 0;
     auto put = [&](const void *src, size_t bytes, size_t span) {
@@ -271,7 +317,8 @@ int build_wmech(ohc_ctx *c) {
     const size_t o_sp = put(sp.data(), sp.size() * 8, b_sp), o_rh = put(rh.data(), rh.size() * 4, b_rh),
                  o_rd = put(rd.data(), rd.size() * 8, b_rd), o_ef = put(eff.data(), eff.size() * 8, b_ef),
                  o_et = put(efft.data(), efft.size() * 8, b_et),
-                 o_pr = put(pair.data(), pair.size() * 8, b_pr);
+                 o_pr = put(pair.data(), pair.size() * 8, b_pr),
+                 o_rc = put(rec.data(), rec.size() * 8, b_rc);
     HIPCHK(c, hipMalloc(&c->d_wm, total));
     HIPCHK(c, hipMemcpy(c->d_wm, h.data(), total, hipMemcpyHostToDevice));
     unsigned char *d = (unsigned char *)c->d_wm;
@@ -284,6 +331,7 @@ int build_wmech(ohc_ctx *c) {
     c->wm.eff = (const double *)(d + o_ef);
     c->wm.efft = (const double *)(d + o_et);
     c->pair.t = (const double *)(d + o_pr);
+    c->src.rec = rec_ok ? (const double *)(d + o_rc) : nullptr;
     return OHC_OK;
 }
 
@@ -828,6 +876,8 @@ int ohc_chem_source(ohc_ctx *c, int64_t n, const double *T, const double *p, con
                          (const double *)dY, ldY, (double *)dR, ldR, (double *)dD, ldD,
                          withoutLastSpec, c->opts.jacobian};
     if (c->lane) HIPCHK(c, c->lane->source(P, c->stream));
+    else if (c->src.rec && std::max(n, c->sliced_n) >= ohcd::kSourceTableMin)
+        HIPCHK(c, ohcd::table_source(P, c->wm, c->src, c->stream));
     else HIPCHK(c, ohcd::wave_source(P, c->wm, c->stream));
     return st.finish();
 }

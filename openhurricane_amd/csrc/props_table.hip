@@ -27,34 +27,9 @@ namespace ohcd {
 
 namespace {
 
-// Tables in the constant address space: wave-uniform reads become scalar
-// loads although the kernels store to global memory in the same loop.
-typedef const __attribute__((address_space(4))) double ctab;
-__device__ __forceinline__ ctab *as_ctab(const double *p) { return (ctab *)(uintptr_t)p; }
-
-// cp0 and ha of species k per unit mass (JANAF.cpp:155-189) with wave-uniform
-// coefficients: both ranges evaluated, the lane's picked
-__device__ __forceinline__ void species_cp_h(ctab *S, int k, double T, double &cp,
-                                             double &h) {
-    const double Tl = S[SP_TLOW * 64 + k], Th = S[SP_THIGH * 64 + k];
-    const double Tx = fmin(fmax(T, Tl), Th);
-    double c[2], e[2];
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        ctab *a = S + (r ? SP_AHI : SP_ALO) * 64 + k, *q = S + (r ? SP_HHI : SP_HLO) * 64 + k;
-        c[r] = (((a[4 * 64] * Tx + a[3 * 64]) * Tx + a[2 * 64]) * Tx + a[64]) * Tx + a[0];
-        e[r] = ((((q[0] * Tx + q[64]) * Tx + q[2 * 64]) * Tx + q[3 * 64]) * Tx + a[0]) * Tx + a[5 * 64];
-    }
-    const bool lo = T < S[SP_TCOM * 64 + k];
-    cp = lo ? c[0] : c[1];
-    h = fma(cp, T - Tx, lo ? e[0] : e[1]);  // linear outside [Tlow, Thigh]
-}
-
 template <int NSP>
 __global__ __launch_bounds__(64, NSP <= 32 ? 3 : 1) void props_table_kernel(const PropParams P, const WMech M,
                                                          const PairTab pt) {
-    // up to 32 species x, x b and x b^2 fit the registers; above, x and b, with
-    // one more multiplication per pair
     // x, x b and x b^2 in registers up to 16 species; above, x and b, with one
     // more multiplication per pair, so that three wavefronts share a SIMD and hide the
     // scalar loads of the rows (32 species, 262,147 cells: 514 us with x, x b, x b^2

@@ -31,6 +31,31 @@ struct PairTab {
     static constexpr int kRow = 8 * 4 * 8;
     const double *t;
 };
+// One record per reaction for kernels with a wave-uniform reaction
+// (source_table.hip).  32-bit words: the packed header (RH_HDR) with flags, the
+// participants' rows (reactants 0..2, products 3..5; species * 64, two to a
+// word; the row past the species for an absent one), their signed coefficients
+// (0 if absent), orders (1 if absent) and the sum of the coefficients; then
+// doubles: the forward, low-pressure and explicit reverse Arrhenius triples, the
+// fall-off parameters, the participants' third-body efficiencies and the
+// reaction's NASA-7 coefficients sum nu_k W_k a_k (low range, high range).
+struct SrcTab {
+    enum { kHdr, kRow, kNu = kRow + 3, kOrd = kNu + 6, kSum = kOrd + 6, kWords = 18 };
+    enum { kArr = kWords / 2, kLow = kArr + 3, kRev = kLow + 3, kFop = kRev + 3, kEff = kFop + 5,
+           kNasa = kEff + 6, kRec = 48 };
+    // header flags: a species on both sides, a third participant on a side, and
+    // (3 bits) the participant that is the last species (7: none)
+    static constexpr unsigned kBoth = 1u << 20, kThree = 1u << 21;
+    static constexpr int kLast = 22;
+    const double *rec;
+    int first_tb;  // first reaction of the table with a third body (they come last)
+};
+// source terms of run-time tables whose coefficients and orders the packed
+// fields hold exactly, with one Tcommon for all species and ns <= 56, for calls
+// of at least kSourceTableMin cells (below, one wavefront per cell is faster: the
+// two cost the same at about 6,000 cells of 32 or 54 species)
+constexpr int64_t kSourceTableMin = 8192;
+hipError_t table_source(const SourceParams &p, const WMech &m, const SrcTab &t, hipStream_t s);
 // mixture thermo / transport and T from h for run-time tables; wave_props is
 // the split-precision form
 hipError_t table_props(const PropParams &p, const WMech &m, const PairTab &pt, hipStream_t s);

@@ -139,6 +139,29 @@ __device__ __forceinline__ WMech wave_mech() {
     return M;
 }
 
+// Tables in the constant address space: wave-uniform reads become scalar
+// loads although a kernel stores to global memory in the same loop.
+typedef const __attribute__((address_space(4))) double ctab;
+__device__ __forceinline__ ctab *as_ctab(const double *p) { return (ctab *)(uintptr_t)p; }
+
+// cp0 and ha of species k per unit mass (JANAF.cpp:155-189) with wave-uniform
+// coefficients: both ranges evaluated, the lane's picked
+__device__ __forceinline__ void species_cp_h(ctab *S, int k, double T, double &cp,
+                                             double &h) {
+    const double Tl = S[SP_TLOW * 64 + k], Th = S[SP_THIGH * 64 + k];
+    const double Tx = fmin(fmax(T, Tl), Th);
+    double c[2], e[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        ctab *a = S + (r ? SP_AHI : SP_ALO) * 64 + k, *q = S + (r ? SP_HHI : SP_HLO) * 64 + k;
+        c[r] = (((a[4 * 64] * Tx + a[3 * 64]) * Tx + a[2 * 64]) * Tx + a[64]) * Tx + a[0];
+        e[r] = ((((q[0] * Tx + q[64]) * Tx + q[2 * 64]) * Tx + q[3 * 64]) * Tx + a[0]) * Tx + a[5 * 64];
+    }
+    const bool lo = T < S[SP_TCOM * 64 + k];
+    cp = lo ? c[0] : c[1];
+    h = fma(cp, T - Tx, lo ? e[0] : e[1]);  // linear outside [Tlow, Thigh]
+}
+
 // Reads of the per-reaction tables through buffer resources: the lane is
 // the one vector offset, the chunk and field a scalar offset, so a table read
 // needs no vector address arithmetic.  Reads past a table return zero.
