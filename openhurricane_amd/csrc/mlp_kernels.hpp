@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace ohcm {
 
@@ -64,118 +65,169 @@ struct GemmArgs {
     const float *bias;  // [N]
     const float *Z;     // EPI_GELU_BWD: saved pre-activation, ld ldc
     // split-K (EPI_F32 only): block z reduces k in [z kc, min(K, (z+1) kc))
-    // into C32 + z zstride; splitk_sum then adds the partial tiles in order
+    // into C32 + z zstride; splitk_sum then adds the partial results in order
     int kc;
     int64_t zstride;
+    float *rowsum;  // EPI_F32: sum over k of A(m, k), at rowsum + z zstride (nullable)
 };
 
-constexpr int kTM = 64, kTN = 64, kTK = 32, kLdsK = kTK + 8;  // +8: LDS row padding
+constexpr int kTM = 64, kTN = 128, kTK = 64, kLdsK = kTK + 8;  // +8: LDS row padding
+
+// Part of an operand tile in a thread's registers, on its way from global
+// memory to LDS as [row][k].  KC: the operand is K-contiguous, and a thread
+// moves 16-byte pieces of rows; else rows are contiguous and a thread moves
+// blocks of 8 k x 8 rows, transposed in registers (two byte permutes per
+// four values; neighbouring threads take neighbouring k, so that their LDS
+// rows fall into different banks).  T0: the thread that takes the first piece.  Loads are 16 bytes wide where base and leading dimension
+// allow and the piece lies inside, else by element; outside the matrix they
+// give zero.
+template <bool KC, int R, int T0 = 0>
+struct Stage {
+    static constexpr int kPieces = KC ? R * kTK / 8 : R * kTK / 64;
+    static constexpr int kPer = (kPieces + 255) / 256, kVec = KC ? 1 : 8;
+    uint4 v[kPer][kVec];
+
+    static __device__ __forceinline__ uint4 row8(const bf16_t *p, int left, bool wide) {
+        if (wide && left >= 8) return *(const uint4 *)p;
+        union {
+            bf16_t h[8];
+            uint4 q;
+        } u;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) u.h[e] = e < left ? p[e] : (bf16_t)0;
+        return u.q;
+    }
+    // rows r0.. of [0, rows), k in [k0, ke)
+    __device__ __forceinline__ void load(const bf16_t *X, int64_t ld, bool wide, int rows, int r0,
+                                         int k0, int ke) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int c = ((threadIdx.x + 256 - T0) & 255) + 256 * i;
+            if (kPieces % 256 != 0 && c >= kPieces) break;
+            if constexpr (KC) {
+                const int r = r0 + c / (kTK / 8), k = k0 + c % (kTK / 8) * 8;
+                v[i][0] = r < rows ? row8(X + (int64_t)r * ld + k, ke - k, wide) : uint4{0, 0, 0, 0};
+            } else {
+                const int r = r0 + c / (kTK / 8) * 8, k = k0 + c % (kTK / 8) * 8;
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    v[i][e] = k + e < ke ? row8(X + (int64_t)(k + e) * ld + r, rows - r, wide)
+                                         : uint4{0, 0, 0, 0};
+            }
+        }
+    }
+    __device__ __forceinline__ void store(bf16_t (*s)[kLdsK]) const {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int c = ((threadIdx.x + 256 - T0) & 255) + 256 * i;
+            if (kPieces % 256 != 0 && c >= kPieces) break;
+            if constexpr (KC) {
+                *(uint4 *)&s[c / (kTK / 8)][c % (kTK / 8) * 8] = v[i][0];
+            } else {
+                const int r = c / (kTK / 8) * 8, k = c % (kTK / 8) * 8;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    uint4 o;
+                    unsigned *w = (unsigned *)&o;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        w[j] = __builtin_amdgcn_perm(((const unsigned *)&v[i][2 * j + 1])[e / 2],
+                                                     ((const unsigned *)&v[i][2 * j])[e / 2],
+                                                     e % 2 ? 0x07060302u : 0x05040100u);
+                    *(uint4 *)&s[r + e][k] = o;
+                }
+            }
+        }
+    }
+};
 
 // C[M x N] = A[M x K] B[K x N] with a fused epilogue.  A 256-thread block
-// computes a 64 x 64 tile (each wavefront a 32 x 32 MFMA tile), staging
-// 64 x 32 slices of A and B through LDS as [row][k]; operands whose rows are
-// not K-contiguous are transposed on the way in.  Edges are zero-padded.
+// computes a 64 x 128 tile (each wavefront two 32 x 32 MFMA tiles) from 64-wide
+// slices of A and B in LDS; the next slice is on its way to registers while
+// the current one is multiplied.  The training batch (16,384 x 256 x 256)
+// gives 512 blocks, two per CU.  Bound by the traffic of its outputs (34 MB
+// with the saved pre-activation) and the latency of the few slices: 17 us
+// forward, 49 us with 64 x 64 tiles and element-wise loads.
 template <bool A_KC, bool B_KC, int EPI>
 __global__ __launch_bounds__(256) void gemm_bf16(const GemmArgs g) {
-    __shared__ bf16_t sA[kTM][kLdsK], sB[kTN][kLdsK];
+    __shared__ __attribute__((aligned(16))) bf16_t sA[kTM][kLdsK], sB[kTN][kLdsK];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m0 = blockIdx.y * kTM, n0 = blockIdx.x * kTN;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
     const int kb = (int)blockIdx.z * g.kc, ke = min(g.K, kb + g.kc);
-    f32x16 acc = {};
+    const bool wa = g.lda % 8 == 0 && (uintptr_t)g.A % 16 == 0,
+               wb = g.ldb % 8 == 0 && (uintptr_t)g.B % 16 == 0;
+    const bool sums = EPI == EPI_F32 && g.rowsum && blockIdx.x == 0;
+    Stage<A_KC, kTM> ra;
+    Stage<B_KC, kTN, B_KC ? 0 : 128> rb;
+    f32x16 acc[2] = {};
+    float rs = 0.0f;
+    ra.load(g.A, g.lda, wa, g.M, m0, kb, ke);
+    rb.load(g.B, g.ldb, wb, g.N, n0, kb, ke);
     for (int k0 = kb; k0 < ke; k0 += kTK) {
-        // ---- stage A and B slices (256 threads x 8 elements each) ----
-        {
-            bf16_t va[8], vb[8];
-            if (A_KC) {
-                const int r = tid >> 2, kk = (tid & 3) * 8;
-                const int m = m0 + r;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int k = k0 + kk + e;
-                    va[e] = (m < g.M && k < ke) ? g.A[(int64_t)m * g.lda + k] : (bf16_t)0;
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) sA[r][kk + e] = va[e];
-            } else {
-                const int kk = tid >> 3, r = (tid & 7) * 8;
-                const int k = k0 + kk;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int m = m0 + r + e;
-                    va[e] = (m < g.M && k < ke) ? g.A[(int64_t)k * g.lda + m] : (bf16_t)0;
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) sA[r + e][kk] = va[e];
-            }
-            if (B_KC) {
-                const int r = tid >> 2, kk = (tid & 3) * 8;
-                const int n = n0 + r;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int k = k0 + kk + e;
-                    vb[e] = (n < g.N && k < ke) ? g.B[(int64_t)n * g.ldb + k] : (bf16_t)0;
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) sB[r][kk + e] = vb[e];
-            } else {
-                const int kk = tid >> 3, r = (tid & 7) * 8;
-                const int k = k0 + kk;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int n = n0 + r + e;
-                    vb[e] = (n < g.N && k < ke) ? g.B[(int64_t)k * g.ldb + n] : (bf16_t)0;
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) sB[r + e][kk] = vb[e];
-            }
-        }
         __syncthreads();
-        // ---- two 32x32x16 MFMA steps per slice ----
+        ra.store(sA);
+        rb.store(sB);
+        __syncthreads();
+        if (k0 + kTK < ke) {
+            ra.load(g.A, g.lda, wa, g.M, m0, k0 + kTK, ke);
+            rb.load(g.B, g.ldb, wb, g.N, n0, k0 + kTK, ke);
+        }
+        const int i = lane & 31, kh = 8 * (lane >> 5);
 #pragma unroll
         for (int ks = 0; ks < kTK; ks += 16) {
-            const int i = lane & 31, kb = ks + 8 * (lane >> 5);
-            bf16x8 a, b;
+            const bf16x8 a = *(const bf16x8 *)&sA[wm + i][ks + kh];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                a[e] = __builtin_bit_cast(__bf16, sA[wm + i][kb + e]);
-                b[e] = __builtin_bit_cast(__bf16, sB[wn + i][kb + e]);
+            for (int c = 0; c < 2; ++c) {
+                const bf16x8 b = *(const bf16x8 *)&sB[wn + 32 * c + i][ks + kh];
+                acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[c], 0, 0, 0);
             }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
         }
-        __syncthreads();
+        if (sums) {  // four threads to a row, 16 k each
+#pragma unroll
+            for (int e = 0; e < 16; ++e) rs += bf2f(sA[tid >> 2][(tid & 3) * 16 + e]);
+        }
     }
     // ---- epilogue ----
-    const int j = n0 + wn + (lane & 31);
+    if (sums) {
+        rs += __shfl_xor(rs, 1);
+        rs += __shfl_xor(rs, 2);
+        const int m = m0 + (tid >> 2);
+        if ((tid & 3) == 0 && m < g.M) g.rowsum[m + (int64_t)blockIdx.z * g.zstride] = rs;
+    }
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int i = m0 + wm + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
-        if (i >= g.M || j >= g.N) continue;
-        const int64_t o = (int64_t)i * g.ldc + j;
-        const float x = acc[v];
-        if (EPI == EPI_F32) {
-            g.C32[o + (int64_t)blockIdx.z * g.zstride] = x;
-        } else if (EPI == EPI_BIAS_F32) {
-            g.C32[o] = x + g.bias[j];
-        } else if (EPI == EPI_BIAS_GELU) {
-            const float z = x + g.bias[j];
-            if (g.C32) g.C32[o] = z;
-            g.C16[o] = f2bf(gelu(z));
-        } else {
-            g.C16[o] = f2bf(x * gelu_grad(g.Z[o]));
+    for (int c = 0; c < 2; ++c) {
+        const int j = n0 + wn + 32 * c + (lane & 31);
+        if (j >= g.N) continue;
+        const float bias = EPI == EPI_BIAS_F32 || EPI == EPI_BIAS_GELU ? g.bias[j] : 0.0f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int i = m0 + wm + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
+            if (i >= g.M) continue;
+            const int64_t o = (int64_t)i * g.ldc + j;
+            const float x = acc[c][v];
+            if (EPI == EPI_F32) {
+                g.C32[o + (int64_t)blockIdx.z * g.zstride] = x;
+            } else if (EPI == EPI_BIAS_F32) {
+                g.C32[o] = x + bias;
+            } else if (EPI == EPI_BIAS_GELU) {
+                const float z = x + bias;
+                if (g.C32) g.C32[o] = z;
+                g.C16[o] = f2bf(gelu(z));
+            } else {
+                g.C16[o] = f2bf(x * gelu_grad(g.Z[o]));
+            }
         }
     }
 }
 
-// C[i][j] = sum over z = 0..S-1, in that order, of the split-K partial tiles.
-__global__ void splitk_sum(int S, int M, int N, int64_t ldc, int64_t zstride, const float *part,
-                           float *C) {
+// G[e] = sum over z = 0..S-1, in that order, of the split-K partial gradients.
+__global__ void splitk_sum(int S, int64_t np, const float *part, float *G) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (int64_t)M * N) return;
-    const int64_t o = (e / N) * ldc + e % N;
-    float v = part[o];
-    for (int z = 1; z < S; ++z) v += part[z * zstride + o];
-    C[o] = v;
+    if (e >= np) return;
+    float v = part[e];
+    for (int z = 1; z < S; ++z) v += part[z * np + e];
+    G[e] = v;
 }
 
 // ---- element-wise training helpers ----
@@ -192,8 +244,9 @@ __global__ void normalize_in(int64_t n, int nin, int kpad, const float *X, const
 
 // Weighted mean-square loss on normalised targets t = (Yt - mean) / std:
 // loss = sum w_k (out - t)^2 / n, dOut = 2 w (out - t) / n (BF16 for the
-// backward GEMMs); per-block partial losses into part[].
-__global__ void loss_grad(int64_t n, int nout, const float *out, const float *Yt,
+// backward GEMMs, rows padded with zeros to ld); per-block partial losses
+// into part[].
+__global__ void loss_grad(int64_t n, int nout, int ld, const float *out, const float *Yt,
                           const float *mean, const float *rstd, const float *w, bf16_t *dOut,
                           float *part) {
     __shared__ float red[256];
@@ -203,7 +256,9 @@ __global__ void loss_grad(int64_t n, int nout, const float *out, const float *Yt
         const int k = (int)(e % nout);
         const float r = out[e] - (Yt[e] - mean[k]) * rstd[k];
         l = w[k] * r * r / (float)n;
-        dOut[e] = f2bf(2.0f * w[k] * r / (float)n);
+        const int64_t i = e / nout;
+        dOut[i * ld + k] = f2bf(2.0f * w[k] * r / (float)n);
+        if (k < ld - nout) dOut[i * ld + nout + k] = (bf16_t)0;
     }
     red[threadIdx.x] = l;
     __syncthreads();
@@ -212,31 +267,6 @@ __global__ void loss_grad(int64_t n, int nout, const float *out, const float *Yt
         __syncthreads();
     }
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-// Column sums db[j] = sum_i dZ[i][j] in two deterministic passes: block
-// (x, y) sums rows [y*kRowChunk, ...) of columns [64x, 64x+64) into
-// part[y][j]; colsum_finish adds the partials in chunk order.
-constexpr int kRowChunk = 256;
-__global__ __launch_bounds__(256) void colsum_partial(int64_t n, int N, int64_t ld,
-                                                      const bf16_t *dZ, float *part) {
-    __shared__ float red[4][64];
-    const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int j = blockIdx.x * 64 + c;
-    const int64_t r0 = (int64_t)blockIdx.y * kRowChunk;
-    float s = 0.0f;
-    if (j < N)
-        for (int64_t i = r0 + q; i < r0 + kRowChunk && i < n; i += 4) s += bf2f(dZ[i * ld + j]);
-    red[q][c] = s;
-    __syncthreads();
-    if (q == 0 && j < N) part[(int64_t)blockIdx.y * N + j] = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
-}
-__global__ void colsum_finish(int nchunk, int N, const float *part, float *db) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= N) return;
-    float s = 0.0f;
-    for (int y = 0; y < nchunk; ++y) s += part[(int64_t)y * N + j];
-    db[j] = s;
 }
 
 // Adam on the flat FP32 master parameters (c1 = 1/(1-b1^t), c2 = 1/(1-b2^t)),
@@ -351,21 +381,86 @@ struct InferArgs {
 
 // network output k (denormalised) -> increment: identity, or the inverse of
 // z = sign(d) ln(1 + |d| / delta_k)
-__device__ __forceinline__ float out_increment(const InferArgs &a, const float *o, int k) {
-    const float z = o[k] * a.out_std[k] + a.out_mean[k];
+// (nrm: output mean, standard deviation and target scale, each [NOUTP])
+template <int NOUTP>
+__device__ __forceinline__ float out_increment(const InferArgs &a, const float (*nrm)[NOUTP],
+                                               const float *o, int k) {
+    const float z = o[k] * nrm[1][k] + nrm[0][k];
     if (!a.delta) return z;
-    return copysignf(expm1f(fabsf(z)), z) * a.delta[k];
+    return copysignf(expm1f(fabsf(z)), z) * nrm[2][k];
 }
 
-// Hidden layer: out[TM][W] = gelu(in[TM][K] W^T + b), 4 wavefronts each
-// producing TM rows x W/4 columns.  IN8: FP8 activations and weights on the
+template <int B, int E, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
+    }
+}
+
+// gelu() for the inference epilogue: the quotient 2 / (1 + e) by the refined
+// reciprocal and a remainder step, as an IEEE division without its scaling (the
+// divisor is at least 1, and clamped below overflow, where the quotient no
+// longer changes 1 - q).
+__device__ __forceinline__ float gelu_fast(float x) {
+    const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+    const float d = fminf(1.0f + __builtin_amdgcn_exp2f(u * 2.885390082f), 1.0e38f);  // 2 / ln 2
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.0f), r, r);
+    float q = r + r;
+    q = fmaf(fmaf(-d, q, 2.0f), r, q);
+    const float t = 1.0f - q;
+    return 0.5f * x * (1.0f + t);
+}
+// two BF16 values (round to nearest even) in one word, low first
+__device__ __forceinline__ unsigned pk_bf16(float a, float b) {
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+    const bf16x2 v = {(__bf16)a, (__bf16)b};
+    return __builtin_bit_cast(unsigned, v);
+}
+
+// ln x to about 1e-14 relative (x positive and normal; else as log): mantissa
+// m in [sqrt(1/2), sqrt(2)), s = (m - 1) / (m + 1), and the series of
+// 2 artanh(s) to s^19 -- a quarter of the library logarithm's instructions, for
+// features that are rounded to FP32 next.
+__device__ __forceinline__ double log_feature(double x) {
+    double m = __builtin_amdgcn_frexp_mant(x);  // [1/2, 1)
+    int e = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    e -= low ? 1 : 0;
+    const double b = m + 1.0;
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.0), r, r);
+    r = fma(fma(-b, r, 1.0), r, r);
+    const double s = (m - 1.0) * r, z = s * s;
+    double p = 2.0 / 19.0;
+    p = fma(p, z, 2.0 / 17.0);
+    p = fma(p, z, 2.0 / 15.0);
+    p = fma(p, z, 2.0 / 13.0);
+    p = fma(p, z, 2.0 / 11.0);
+    p = fma(p, z, 2.0 / 9.0);
+    p = fma(p, z, 2.0 / 7.0);
+    p = fma(p, z, 2.0 / 5.0);
+    p = fma(p, z, 2.0 / 3.0);
+    p = fma(p, z, 2.0);
+    const double l = fma((double)e, 0.69314718055994530942, s * p);
+    return x > 0.0 ? l : (x == 0.0 ? -__builtin_huge_val() : __builtin_nan(""));
+}
+
+// Hidden layer: out[TM][W] = gelu(in[TM][K] W^T + b), NW wavefronts each
+// producing TM rows x W/NW columns.  IN8: FP8 activations and weights on the
 // 32x32x64 f8f6f4 MFMA (unit block scales; per-row weight scale applied in
 // the epilogue), else BF16 on 32x32x16.  OUT8: the epilogue writes FP8.
-// Strides LDI / LDO count elements of the buffer's type.
-template <int TM, int WD, int K, int LDI, int LDO, bool IN8, bool OUT8>
+// Strides LDI / LDO count elements of the buffer's type.  The weights are the
+// first MFMA operand, so that a lane's accumulators hold four consecutive
+// features of one cell at a time: the epilogue packs and stores them as one
+// word or two.  The layer is bound by that epilogue (24 vector instructions per
+// activation), not by the matrix cores.
+template <int TM, int WD, int NW, int K, int LDI, int LDO, bool IN8, bool OUT8>
 __device__ __forceinline__ void mlp_layer(const void *sin_, void *sout_, const void *Wl_,
                                           const float *ws, const float *bl) {
-    constexpr int RT = TM / 32, CT = WD / 128;
+    constexpr int RT = TM / 32, CT = WD / (32 * NW);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     f32x16 acc[RT][CT];
 #pragma unroll
@@ -373,111 +468,155 @@ __device__ __forceinline__ void mlp_layer(const void *sin_, void *sout_, const v
 #pragma unroll
         for (int c = 0; c < CT; ++c) acc[r][c] = f32x16{};
     const int i = lane & 31, h = lane >> 5;
-    if constexpr (IN8) {
-        const uint8_t *sin = (const uint8_t *)sin_, *Wl = (const uint8_t *)Wl_;
+    // The weights come from L2: a group of KG steps' fragments is requested ahead
+    // of the group before it (one wait per group instead of one per step).
+    using W_t = std::conditional_t<IN8, uint8_t, bf16_t>;
+    using frag = std::conditional_t<IN8, i32x8, bf16x8>;
+    constexpr int KS = IN8 ? 64 : 16, NK = K / KS, KW = IN8 ? 32 : 8;  // k of a step, steps, k of a lane
+    constexpr int KG = IN8 ? 2 : (CT > 2 ? 4 : 8);
+    const W_t *sin = (const W_t *)sin_ + i * LDI + KW * h;
+    const W_t *Wl = (const W_t *)Wl_ + (int64_t)(wave * (CT * 32) + i) * K + KW * h;
+    frag b[2][KG][CT];
+    auto load = [&](auto gc) __attribute__((always_inline)) {
+        constexpr int g = gc;
 #pragma unroll
-        for (int k0 = 0; k0 < K; k0 += 64) {
-            i32x8 a[RT], b[CT];
-#pragma unroll
-            for (int r = 0; r < RT; ++r) a[r] = *(const i32x8 *)(sin + (r * 32 + i) * LDI + k0 + 32 * h);
-#pragma unroll
-            for (int c = 0; c < CT; ++c) {
-                const int nn = wave * (CT * 32) + c * 32 + i;
-                b[c] = *(const i32x8 *)(Wl + (int64_t)nn * K + k0 + 32 * h);
-            }
-#pragma unroll
-            for (int r = 0; r < RT; ++r)
-#pragma unroll
-                for (int c = 0; c < CT; ++c)
-                    acc[r][c] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                        a[r], b[c], acc[r][c], 0, 0, 0, 127, 0, 127);
-        }
-    } else {
-        const bf16_t *sin = (const bf16_t *)sin_, *Wl = (const bf16_t *)Wl_;
-        const int kh = 8 * h;
-#pragma unroll
-        for (int k0 = 0; k0 < K; k0 += 16) {
-            bf16x8 a[RT], b[CT];
-#pragma unroll
-            for (int r = 0; r < RT; ++r) a[r] = *(const bf16x8 *)(sin + (r * 32 + i) * LDI + k0 + kh);
-#pragma unroll
-            for (int c = 0; c < CT; ++c) {
-                const int nn = wave * (CT * 32) + c * 32 + i;
-                b[c] = *(const bf16x8 *)(Wl + (int64_t)nn * K + k0 + kh);
-            }
-#pragma unroll
-            for (int r = 0; r < RT; ++r)
+        for (int t = 0; t < KG; ++t)
+            if (g * KG + t < NK)
 #pragma unroll
                 for (int c = 0; c < CT; ++c)
-                    acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r], b[c], acc[r][c], 0, 0, 0);
-        }
-    }
+                    b[g % 2][t][c] = *(const frag *)(Wl + (int64_t)c * 32 * K + (g * KG + t) * KS);
+    };
+    load(std::integral_constant<int, 0>{});
+    constexpr int NG = (NK + KG - 1) / KG;
+    auto group = [&](auto gc) __attribute__((always_inline)) {
+        constexpr int g = gc;
+        if constexpr (g + 1 < NG) load(std::integral_constant<int, g + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int c = 0; c < CT; ++c) {
-        const int col = wave * (CT * 32) + c * 32 + i;
-        const float bias = bl[col];
-        const float scale = IN8 ? ws[col] : 1.0f;
+        for (int t = 0; t < KG; ++t)
+            if (g * KG + t < NK) {
+                frag a[RT];
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
+                for (int r = 0; r < RT; ++r)
+                    a[r] = *(const frag *)(sin + r * 32 * LDI + (g * KG + t) * KS);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int row = r * 32 + 8 * (v / 4) + 4 * h + (v % 4);
-                const float g = gelu(acc[r][c][v] * scale + bias);
-                if constexpr (OUT8) ((uint8_t *)sout_)[row * LDO + col] = f2e4m3_hw(g);
-                else ((bf16_t *)sout_)[row * LDO + col] = f2bf(g);
+                for (int r = 0; r < RT; ++r)
+#pragma unroll
+                    for (int c = 0; c < CT; ++c) {
+                        if constexpr (IN8)
+                            acc[r][c] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                                b[g % 2][t][c], a[r], acc[r][c], 0, 0, 0, 127, 0, 127);
+                        else
+                            acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[g % 2][t][c], a[r],
+                                                                                acc[r][c], 0, 0, 0);
+                    }
             }
-    }
+    };
+    static_for<0, NG>(group);
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            // features col .. col + 3 of cell r * 32 + i
+            const int col = wave * (CT * 32) + c * 32 + 8 * q + 4 * h;
+            const float4 b4 = *(const float4 *)(bl + col);
+            const float bias[4] = {b4.x, b4.y, b4.z, b4.w};
+            float scale[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+            if constexpr (IN8) {
+                const float4 s4 = *(const float4 *)(ws + col);
+                scale[0] = s4.x, scale[1] = s4.y, scale[2] = s4.z, scale[3] = s4.w;
+            }
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                float g[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    g[e] = gelu_fast(acc[r][c][4 * q + e] * scale[e] + bias[e]);
+                const int o = (r * 32 + i) * LDO + col;
+                if constexpr (OUT8)
+                    *(unsigned *)((uint8_t *)sout_ + o) =
+                        f2e4m3_hw(g[0]) | f2e4m3_hw(g[1]) << 8 | f2e4m3_hw(g[2]) << 16 |
+                        (unsigned)f2e4m3_hw(g[3]) << 24;
+                else
+                    *(uint2 *)((bf16_t *)sout_ + o) = uint2{pk_bf16(g[0], g[1]), pk_bf16(g[2], g[3])};
+            }
+        }
 }
 
-// One block of 256 threads advances TM cells: features (T, log p, log Y) ->
+// One block of NW wavefronts advances TM cells: features (T, log p, log Y) ->
 // normalised BF16 -> hidden layers -> increments (dT, dlog Y) -> new state,
 // gated on the dt match, the input box (OOD), the element-mass change and,
 // with a peer network, the two networks' agreement (the state then takes the
 // mean of both increments).  FP8: the hidden-to-hidden layers run in FP8.
-template <int TM, int WD, int KIN, int NOUTP, bool FP8>
-__global__ __launch_bounds__(256) void mlp_infer(const InferArgs a) {
+template <int TM, int WD, int NW, int KIN, int NOUTP, bool FP8>
+__global__ __launch_bounds__(64 * NW) void mlp_infer(const InferArgs a) {
+    constexpr int NT = 64 * NW;
     constexpr int LD = WD + 8;   // LDS row stride (bf16) of the activation buffers
     constexpr int LD8 = WD + 16; // the same buffers holding FP8 rows (bytes)
     static_assert(TM * LD8 <= TM * LD * 2, "FP8 rows must fit the buffer");
     __shared__ __attribute__((aligned(16))) bf16_t buf[2][TM * LD];
     __shared__ int sfail[TM];
+    __shared__ float snorm[4][KIN], sout_n[3][NOUTP];  // input / output normalisation
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t c0 = (int64_t)blockIdx.x * TM;
     const int nin = a.ns + 2, nout = a.ns + 1;
     if (tid < TM) sfail[tid] = 0;
+    for (int e = tid; e < 4 * KIN; e += NT) {
+        const int q = e / KIN, k = e % KIN;
+        const float *src = q == 0 ? a.in_mean : q == 1 ? a.in_rstd : q == 2 ? a.zlo : a.zhi;
+        snorm[q][k] = k < nin ? src[k] : 0.0f;
+    }
+    for (int e = tid; e < 3 * NOUTP; e += NT) {
+        const int q = e / NOUTP, k = e % NOUTP;
+        const float *src = q == 0 ? a.out_mean : q == 1 ? a.out_std : a.delta;
+        sout_n[q][k] = k < nout && src ? src[k] : 0.0f;
+    }
     __syncthreads();
     // ---- features, normalised, into buf[0] as [TM][KIN] (stride LD) ----
-    for (int e = tid; e < TM * KIN; e += 256) {
-        const int k = e / TM, r = e % TM;
-        const int64_t cell = c0 + r;
-        float z = 0.0f;
-        if (k < nin && cell < a.n) {
-            double x;
-            if (k == 0) x = a.T[cell];
-            else if (k == 1) x = log(a.p[cell]);
-            else x = log(fmax(a.Y[(int64_t)(k - 2) * a.ldY + cell], kYFloor));
-            z = ((float)x - a.in_mean[k]) * a.in_rstd[k];
-            if (!(z >= a.zlo[k] && z <= a.zhi[k])) atomicOr(&sfail[r], 1);
+    // Thread tid takes the features tid / TM + m (256 / TM) of cell tid % TM, all
+    // loads first; normalisation and box come from LDS and the box check is one flag
+    // per thread (with four table loads and a branch per value the features took
+    // 42 k of a block's 97 k cycles).
+    {
+        constexpr int IT = TM * KIN / NT, KT = NT / TM;
+        const int r = tid % TM, k0 = tid / TM;
+        const bool in = c0 + r < a.n;
+        const int64_t cell = in ? c0 + r : a.n - 1;
+        double v[IT];
+#pragma unroll
+        for (int m = 0; m < IT; ++m) {
+            const int k = k0 + KT * m;
+            const double *src = k == 0 ? a.T : k == 1 ? a.p : a.Y + (int64_t)min(k - 2, a.ns - 1) * a.ldY;
+            v[m] = src[cell];
         }
-        buf[0][r * LD + k] = f2bf(z);
+        bool ood = false;
+#pragma unroll
+        for (int m = 0; m < IT; ++m) {
+            const int k = k0 + KT * m;
+            const double l = log_feature(k == 1 ? v[m] : fmax(v[m], kYFloor));
+            const float z = ((float)(k == 0 ? v[m] : l) - snorm[0][k]) * snorm[1][k];
+            ood = ood || (k < nin && !(z >= snorm[2][k] && z <= snorm[3][k]));
+            buf[0][r * LD + k] = f2bf(k < nin && in ? z : 0.0f);
+        }
+        if (ood && in) atomicOr(&sfail[r], 1);
     }
     __syncthreads();
     // ---- hidden layers (ping-pong between the two buffers) ----
     const bool l1_fp8 = FP8 && a.depth > 1;
-    if (l1_fp8) mlp_layer<TM, WD, KIN, LD, LD8, false, true>(buf[0], buf[1], a.W + a.woff[0], nullptr, a.b + a.boff[0]);
-    else mlp_layer<TM, WD, KIN, LD, LD, false, false>(buf[0], buf[1], a.W + a.woff[0], nullptr, a.b + a.boff[0]);
+    if (l1_fp8) mlp_layer<TM, WD, NW, KIN, LD, LD8, false, true>(buf[0], buf[1], a.W + a.woff[0], nullptr, a.b + a.boff[0]);
+    else mlp_layer<TM, WD, NW, KIN, LD, LD, false, false>(buf[0], buf[1], a.W + a.woff[0], nullptr, a.b + a.boff[0]);
     __syncthreads();
     int cur = 1;
     for (int l = 1; l < a.depth; ++l) {
         if constexpr (FP8) {
             if (l + 1 < a.depth)
-                mlp_layer<TM, WD, WD, LD8, LD8, true, true>(buf[cur], buf[cur ^ 1], a.W8 + a.w8off[l],
+                mlp_layer<TM, WD, NW, WD, LD8, LD8, true, true>(buf[cur], buf[cur ^ 1], a.W8 + a.w8off[l],
                                                              a.s8 + a.s8off[l], a.b + a.boff[l]);
             else
-                mlp_layer<TM, WD, WD, LD8, LD, true, false>(buf[cur], buf[cur ^ 1], a.W8 + a.w8off[l],
+                mlp_layer<TM, WD, NW, WD, LD8, LD, true, false>(buf[cur], buf[cur ^ 1], a.W8 + a.w8off[l],
                                                              a.s8 + a.s8off[l], a.b + a.boff[l]);
         } else {
-            mlp_layer<TM, WD, WD, LD, LD, false, false>(buf[cur], buf[cur ^ 1], a.W + a.woff[l],
+            mlp_layer<TM, WD, NW, WD, LD, LD, false, false>(buf[cur], buf[cur ^ 1], a.W + a.woff[l],
                                                          nullptr, a.b + a.boff[l]);
         }
         __syncthreads();
@@ -490,6 +629,7 @@ __global__ __launch_bounds__(256) void mlp_infer(const InferArgs a) {
     {
         constexpr int RT = TM / 32, CTO = NOUTP / 32;
         const int i = lane & 31, kh = 8 * (lane >> 5);
+        static_assert(RT * CTO <= NW, "one wavefront per output tile");
         if (wave < RT * CTO) {
             const int r = wave / CTO, c = wave % CTO;
             const bf16_t *Wl = a.W + a.woff[a.depth];
@@ -509,20 +649,23 @@ __global__ __launch_bounds__(256) void mlp_infer(const InferArgs a) {
         }
     }
     __syncthreads();
+    if (a.mode == 1) {
+        // the block's increments are contiguous: element e of [TM][nout] per thread
+        const int ne = (int)min((int64_t)TM, a.n - c0) * nout;
+        for (int e = tid; e < ne; e += NT)
+            a.out32[c0 * nout + e] = out_increment<NOUTP>(a, sout_n, sout + (e / nout) * LDF, e % nout);
+        return;
+    }
     // ---- per cell: increments, new state, gate ----
     if (tid >= TM) return;
     const int64_t cell = c0 + tid;
     if (cell >= a.n) return;
     const float *o = sout + tid * LDF;
-    if (a.mode == 1) {
-        for (int k = 0; k < nout; ++k) a.out32[cell * nout + k] = out_increment(a, o, k);
-        return;
-    }
     bool ok = sfail[tid] == 0;
     ok = ok && fabs(a.dt[cell] * a.dtFactor - a.dt_train) <= 1e-9 * a.dt_train;
     const double T0 = a.T[cell];
     const float *q = a.peer ? a.peer + cell * nout : nullptr;
-    double dT = out_increment(a, o, 0);
+    double dT = out_increment<NOUTP>(a, sout_n, o, 0);
     if (q) {
         ok = ok && fabs(dT - (double)q[0]) <= a.peer_tol * T0;
         dT = 0.5 * (dT + (double)q[0]);
@@ -537,7 +680,7 @@ __global__ __launch_bounds__(256) void mlp_infer(const InferArgs a) {
     for (int k = 0; k < a.ns; ++k) {
         const double yk = a.Y[(int64_t)k * a.ldY + cell];
         const double y0 = fmax(yk, kYFloor);
-        const double ds = out_increment(a, o, k + 1);
+        const double ds = out_increment<NOUTP>(a, sout_n, o, k + 1);
         const double dq = q ? (double)q[k + 1] : ds;
         const double d = q ? 0.5 * (ds + dq) : ds;
         const double v = y0 * exp(d);

@@ -120,8 +120,8 @@ struct ohc_surrogate {
     bf16_t *X16 = nullptr, *dOut = nullptr, *dZa = nullptr, *dZb = nullptr;
     std::vector<float *> Z;
     std::vector<bf16_t *> H;
-    float *out = nullptr, *part = nullptr, *part2 = nullptr, *lsum = nullptr;
-    float *wsplit = nullptr;  // split-K partial tiles of the weight gradients
+    float *out = nullptr, *part = nullptr, *lsum = nullptr;
+    float *wsplit = nullptr;  // split-K partial gradients, [split][parameter]
     int *d_fail = nullptr;
     unsigned int *d_nfail = nullptr;
     int64_t fail_cap = 0;
@@ -135,7 +135,14 @@ float *nm(ohc_surrogate *s, int which) {  // 0..3 in_*, 4..7 out_*
     return s->d_norm + off[which];
 }
 
-constexpr int kMaxSplit = 16;  // split-K factor limit of the weight-gradient GEMMs
+// Split-K factor of the weight-gradient GEMMs of a batch of B rows: they
+// reduce over the batch into a few tiles, so K is split until the launch fills
+// the chip, at least 512 rows to a split.
+constexpr int kMaxSplit = 32;
+int wgrad_split(int64_t B) { return (int)std::min<int64_t>(kMaxSplit, std::max<int64_t>(1, B / 512)); }
+// leading dimensions of the padded activations (16-byte rows)
+int ld_in(const ohc_surrogate *s) { return rup(s->nin, 8); }
+int ld_out(const ohc_surrogate *s) { return rup(s->nout, 8); }
 
 int ensure_ws(ohc_surrogate *s, int64_t B) {
     if (B <= s->cap) return OHC_OK;
@@ -146,12 +153,11 @@ int ensure_ws(ohc_surrogate *s, int64_t B) {
     s->cap = 0;
     const int W = s->width;
     auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t bx = al(2 * B * s->nin), bz = al(4 * B * W), bh = al(2 * B * W),
-                 bo = al(4 * B * s->nout), bdo = al(2 * B * s->nout),
-                 bl = al(4 * (size_t)(nblk(B * s->nout) + 64)),
-                 bp = bl + al(4 * (size_t)(B / ohcm::kRowChunk + 2) * std::max(W, s->nout));
-    const size_t bw = al(4 * (size_t)kMaxSplit * W * std::max(std::max(W, s->nin), s->nout));
-    const size_t total = bx + s->depth * (bz + bh) + bo + bdo + 2 * bh + bp + 256 + bw;
+    const size_t bx = al(2 * B * ld_in(s)), bz = al(4 * B * W), bh = al(2 * B * W),
+                 bo = al(4 * B * s->nout), bdo = al(2 * B * ld_out(s)),
+                 bl = al(4 * (size_t)(nblk(B * s->nout) + 64));
+    const size_t bw = al(4 * (size_t)wgrad_split(B) * s->np);
+    const size_t total = bx + s->depth * (bz + bh) + bo + bdo + 2 * bh + bl + 256 + bw;
     HIPCHK(c, hipMalloc(&s->d_ws, total));
     char *q = (char *)s->d_ws;
     s->X16 = (bf16_t *)q;
@@ -175,8 +181,7 @@ int ensure_ws(ohc_surrogate *s, int64_t B) {
     s->lsum = (float *)q;
     q += 256;
     s->part = (float *)q;
-    s->part2 = (float *)(q + bl);
-    q += bp;
+    q += bl;
     s->wsplit = (float *)q;
     s->cap = B;
     return OHC_OK;
@@ -186,46 +191,25 @@ template <bool AK, bool BK, int EPI>
 hipError_t gemm(hipStream_t st, int M, int N, int K, const bf16_t *A, int64_t lda, const bf16_t *B,
                 int64_t ldb, float *C32, bf16_t *C16, int64_t ldc, const float *bias = nullptr,
                 const float *Zs = nullptr) {
-    ohcm::GemmArgs g{M, N, K, A, lda, B, ldb, C32, C16, ldc, bias, Zs, K, 0};
+    ohcm::GemmArgs g{M, N, K, A, lda, B, ldb, C32, C16, ldc, bias, Zs, K, 0, nullptr};
     const dim3 grid((unsigned)((N + ohcm::kTN - 1) / ohcm::kTN), (unsigned)((M + ohcm::kTM - 1) / ohcm::kTM));
     hipLaunchKernelGGL((ohcm::gemm_bf16<AK, BK, EPI>), grid, dim3(256), 0, st, g);
     return hipGetLastError();
 }
 
-// Weight gradients dW = dZ^T H reduce over the batch (K = batch rows) into a
-// few 64 x 64 tiles; split K so that the launch fills the chip, each split
-// writing its own partial tile into ws, then add the partials in a fixed
-// order (deterministic).
-hipError_t gemm_wgrad(hipStream_t st, int M, int N, int K, const bf16_t *A, int64_t lda,
-                      const bf16_t *B, int64_t ldb, float *C32, int64_t ldc, float *ws) {
-    const int gx = (N + ohcm::kTN - 1) / ohcm::kTN, gy = (M + ohcm::kTM - 1) / ohcm::kTM;
-    int S = std::min(kMaxSplit, std::max(1, 256 / (gx * gy)));
-    S = std::min(S, std::max(1, K / 256));  // at least 256 batch rows per split
-    if (S <= 1) return gemm<false, false, ohcm::EPI_F32>(st, M, N, K, A, lda, B, ldb, C32, nullptr, ldc);
-    const int kc = ((K + S - 1) / S + ohcm::kTK - 1) / ohcm::kTK * ohcm::kTK;
-    S = (K + kc - 1) / kc;
-    const int64_t zs = (int64_t)M * ldc;
-    ohcm::GemmArgs g{M, N, K, A, lda, B, ldb, ws, nullptr, ldc, nullptr, nullptr, kc, zs};
-    hipLaunchKernelGGL((ohcm::gemm_bf16<false, false, ohcm::EPI_F32>), dim3(gx, gy, S), dim3(256), 0, st,
-                       g);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(ohcm::splitk_sum, dim3(nblk((int64_t)M * N)), dim3(256), 0, st, S, M, N, ldc,
-                       zs, ws, C32);
+// Weight and bias gradients of one layer, dW = dZ^T H [M x N] and db = column
+// sums of dZ (its rows' sums as the transposed operand): K = batch rows split
+// into S parts, part z writing its result to C + z np (a layer's weights
+// are followed by its biases in the flat layout).  splitk_sum then adds the
+// parts of all layers in a fixed order (deterministic).
+hipError_t gemm_wgrad(hipStream_t st, int M, int N, int K, int S, const bf16_t *dZ, int64_t ldz,
+                      const bf16_t *H, int64_t ldh, float *C, int64_t np) {
+    const int kc = rup((K + S - 1) / S, ohcm::kTK);
+    ohcm::GemmArgs g{M, N, K, dZ, ldz, H, ldh, C, nullptr, N, nullptr, nullptr, kc, np, C + (int64_t)M * N};
+    const dim3 grid((unsigned)((N + ohcm::kTN - 1) / ohcm::kTN),
+                    (unsigned)((M + ohcm::kTM - 1) / ohcm::kTM), (unsigned)S);
+    hipLaunchKernelGGL((ohcm::gemm_bf16<false, false, ohcm::EPI_F32>), grid, dim3(256), 0, st, g);
     return hipGetLastError();
-}
-
-int colsum(ohc_surrogate *s, int64_t n, int N, const bf16_t *dZ, float *db) {
-    ohc_ctx *c = s->ctx;
-    const int nchunk = (int)((n + ohcm::kRowChunk - 1) / ohcm::kRowChunk);
-    float *part = s->part2;
-    hipLaunchKernelGGL(ohcm::colsum_partial, dim3(nblk(N, 64), nchunk), dim3(256), 0, c->stream, n,
-                       N, (int64_t)N, dZ, part);
-    HIPCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(ohcm::colsum_finish, dim3(nblk(N)), dim3(256), 0, c->stream, nchunk, N,
-                       part, db);
-    HIPCHK(c, hipGetLastError());
-    return OHC_OK;
 }
 
 // Forward and backward over a batch of raw features / targets: gradients into
@@ -236,7 +220,8 @@ int forward_backward(ohc_surrogate *s, int64_t n, const float *X, const float *Y
     int rc = ensure_ws(s, n);
     if (rc) return rc;
     const int W = s->width, L = s->depth, nin = s->nin, nout = s->nout;
-    hipLaunchKernelGGL(ohcm::normalize_in, dim3(nblk(n * nin)), dim3(256), 0, st, n, nin, nin, X,
+    const int li = ld_in(s), lo = ld_out(s);
+    hipLaunchKernelGGL(ohcm::normalize_in, dim3(nblk(n * li)), dim3(256), 0, st, n, nin, li, X,
                        nm(s, 0), nm(s, 1), s->X16);
     HIPCHK(c, hipGetLastError());
     const bf16_t *P16 = s->d_p16;
@@ -245,38 +230,44 @@ int forward_backward(ohc_surrogate *s, int64_t n, const float *X, const float *Y
     for (int l = 0; l < L; ++l) {
         const bf16_t *A = l == 0 ? s->X16 : s->H[l - 1];
         const int K = l == 0 ? nin : W;
-        HIPCHK(c, (gemm<true, true, ohcm::EPI_BIAS_GELU>(st, (int)n, W, K, A, K, P16 + s->w_off[l], K,
-                                                         s->Z[l], s->H[l], W, P + s->b_off[l])));
+        HIPCHK(c, (gemm<true, true, ohcm::EPI_BIAS_GELU>(st, (int)n, W, K, A, l == 0 ? li : W,
+                                                         P16 + s->w_off[l], K, s->Z[l], s->H[l], W,
+                                                         P + s->b_off[l])));
     }
     HIPCHK(c, (gemm<true, true, ohcm::EPI_BIAS_F32>(st, (int)n, nout, W, s->H[L - 1], W,
                                                     P16 + s->w_off[L], W, s->out, nullptr, nout,
                                                     P + s->b_off[L])));
     const unsigned nb = nblk(n * nout);
-    hipLaunchKernelGGL(ohcm::loss_grad, dim3(nb), dim3(256), 0, st, n, nout, s->out, Yt, nm(s, 4),
-                       nm(s, 6), nm(s, 7), s->dOut, s->part);
+    hipLaunchKernelGGL(ohcm::loss_grad, dim3(nb), dim3(256), 0, st, n, nout, lo, s->out, Yt,
+                       nm(s, 4), nm(s, 6), nm(s, 7), s->dOut, s->part);
     HIPCHK(c, hipGetLastError());
     hipLaunchKernelGGL(ohcm::sum_partials, dim3(1), dim3(256), 0, st, (int)nb, s->part, s->lsum);
     HIPCHK(c, hipGetLastError());
-    // backward
-    float *G = s->d_g;
-    HIPCHK(c, gemm_wgrad(st, nout, W, (int)n, s->dOut, nout, s->H[L - 1], W, G + s->w_off[L], W,
-                         s->wsplit));
-    if ((rc = colsum(s, n, nout, s->dOut, G + s->b_off[L]))) return rc;
+    // backward: partial gradients of every layer, added at the end
+    const int kc = rup((int)((n + wgrad_split(n) - 1) / wgrad_split(n)), ohcm::kTK);
+    const int S = (int)((n + kc - 1) / kc);  // no empty split
+    float *G = S > 1 ? s->wsplit : s->d_g;
+    HIPCHK(c, gemm_wgrad(st, nout, W, (int)n, S, s->dOut, lo, s->H[L - 1], W, G + s->w_off[L],
+                         s->np));
     bf16_t *dz = s->dZa, *dz2 = s->dZb;
-    HIPCHK(c, (gemm<true, false, ohcm::EPI_GELU_BWD>(st, (int)n, W, nout, s->dOut, nout,
+    HIPCHK(c, (gemm<true, false, ohcm::EPI_GELU_BWD>(st, (int)n, W, nout, s->dOut, lo,
                                                      P16 + s->w_off[L], W, nullptr, dz, W, nullptr,
                                                      s->Z[L - 1])));
     for (int l = L - 1; l >= 0; --l) {
         const bf16_t *Hin = l == 0 ? s->X16 : s->H[l - 1];
-        const int K = l == 0 ? nin : W;
-        HIPCHK(c, gemm_wgrad(st, W, K, (int)n, dz, W, Hin, K, G + s->w_off[l], K, s->wsplit));
-        if ((rc = colsum(s, n, W, dz, G + s->b_off[l]))) return rc;
+        HIPCHK(c, gemm_wgrad(st, W, l == 0 ? nin : W, (int)n, S, dz, W, Hin, l == 0 ? li : W,
+                             G + s->w_off[l], s->np));
         if (l > 0) {
             HIPCHK(c, (gemm<true, false, ohcm::EPI_GELU_BWD>(st, (int)n, W, W, dz, W,
                                                              P16 + s->w_off[l], W, nullptr, dz2, W,
                                                              nullptr, s->Z[l - 1])));
             std::swap(dz, dz2);
         }
+    }
+    if (S > 1) {
+        hipLaunchKernelGGL(ohcm::splitk_sum, dim3(nblk(s->np)), dim3(256), 0, st, S, s->np,
+                           s->wsplit, s->d_g);
+        HIPCHK(c, hipGetLastError());
     }
     return OHC_OK;
 }
@@ -304,26 +295,25 @@ int pack(ohc_surrogate *s) {
     return OHC_OK;
 }
 
-template <int TM, int WD, int KIN, int NOUTP>
+template <int TM, int WD, int NW, int KIN, int NOUTP>
 void launch_infer(bool fp8, const ohcm::InferArgs &a, hipStream_t st) {
-    if (fp8)
-        hipLaunchKernelGGL((ohcm::mlp_infer<TM, WD, KIN, NOUTP, true>), dim3(nblk(a.n, TM)), dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL((ohcm::mlp_infer<TM, WD, KIN, NOUTP, false>), dim3(nblk(a.n, TM)), dim3(256), 0, st, a);
+    const dim3 g(nblk(a.n, TM)), b(64 * NW);
+    if (fp8) hipLaunchKernelGGL((ohcm::mlp_infer<TM, WD, NW, KIN, NOUTP, true>), g, b, 0, st, a);
+    else hipLaunchKernelGGL((ohcm::mlp_infer<TM, WD, NW, KIN, NOUTP, false>), g, b, 0, st, a);
 }
 
-template <int TM, int WD>
+template <int TM, int WD, int NW>
 hipError_t infer_wd(int kin, int noutp, bool fp8, const ohcm::InferArgs &a, hipStream_t st) {
     if (noutp == 32) {
-        if (kin == 16) launch_infer<TM, WD, 16, 32>(fp8, a, st);
-        else if (kin == 32) launch_infer<TM, WD, 32, 32>(fp8, a, st);
-        else if (kin == 48) launch_infer<TM, WD, 48, 32>(fp8, a, st);
-        else launch_infer<TM, WD, 64, 32>(fp8, a, st);
+        if (kin == 16) launch_infer<TM, WD, NW, 16, 32>(fp8, a, st);
+        else if (kin == 32) launch_infer<TM, WD, NW, 32, 32>(fp8, a, st);
+        else if (kin == 48) launch_infer<TM, WD, NW, 48, 32>(fp8, a, st);
+        else launch_infer<TM, WD, NW, 64, 32>(fp8, a, st);
     } else {
-        if (kin == 16) launch_infer<TM, WD, 16, 64>(fp8, a, st);
-        else if (kin == 32) launch_infer<TM, WD, 32, 64>(fp8, a, st);
-        else if (kin == 48) launch_infer<TM, WD, 48, 64>(fp8, a, st);
-        else launch_infer<TM, WD, 64, 64>(fp8, a, st);
+        if (kin == 16) launch_infer<TM, WD, NW, 16, 64>(fp8, a, st);
+        else if (kin == 32) launch_infer<TM, WD, NW, 32, 64>(fp8, a, st);
+        else if (kin == 48) launch_infer<TM, WD, NW, 48, 64>(fp8, a, st);
+        else launch_infer<TM, WD, NW, 64, 64>(fp8, a, st);
     }
     return hipGetLastError();
 }
@@ -360,8 +350,18 @@ int infer(ohc_surrogate *s, ohcm::InferArgs &a) {
     a.T_high = c->opts.T_high;
     if (a.n == 0) return OHC_OK;
     const bool fp8 = s->precision == 1;
-    if (s->width == 256) HIPCHK(c, (infer_wd<64, 256>(s->kin, s->noutp, fp8, a, c->stream)));
-    else HIPCHK(c, (infer_wd<32, 512>(s->kin, s->noutp, fp8, a, c->stream)));
+    // Every block reads the whole network from L2, so large calls take twice the
+    // cells (and wavefronts) to a block where that gains more than the phases of
+    // two smaller blocks on a CU overlapping.  Width 512, 54 species: from one block
+    // per CU on (17,000 cells 121 -> 101 us; 262,144 cells BF16 1,231 -> 809 us, FP8
+    // 1,081 -> 644 us).  Width 256, 32 species: BF16 from four blocks per CU on
+    // (1,048,576 cells 1,115 -> 1,041 us; 33,000 cells 58 -> 66 us), FP8 never (942 ->
+    // 1,020 us: half the weight bytes).  The results do not depend on the tile.
+    const bool big = s->width == 256 ? !fp8 && a.n >= (int64_t)c->cus * 512 : a.n >= (int64_t)c->cus * 64;
+    if (s->width == 256 && big) HIPCHK(c, (infer_wd<128, 256, 8>(s->kin, s->noutp, fp8, a, c->stream)));
+    else if (s->width == 256) HIPCHK(c, (infer_wd<64, 256, 4>(s->kin, s->noutp, fp8, a, c->stream)));
+    else if (big) HIPCHK(c, (infer_wd<64, 512, 8>(s->kin, s->noutp, fp8, a, c->stream)));
+    else HIPCHK(c, (infer_wd<32, 512, 4>(s->kin, s->noutp, fp8, a, c->stream)));
     return OHC_OK;
 }
 
