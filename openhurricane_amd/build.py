@@ -73,7 +73,7 @@ def build(verbose: bool = True) -> Path:
         entries.append(name)
     reg = GEN / "lane_registry.hip"
     lines = ['// Generated by build.py -- registry of specialised lane kernels.',
-             '#include "lane_kernels.hpp"']
+             '#include "lane_kernels.hpp"', '#include "quad_lane.hpp"']
     lines += [f'#include "mech_{n}.h"' for n in entries]
     lines += ["", "static const ohcd::LaneEntry kEntries[] = {"]
     lines += [f'    ohcd::LaneLaunch<Mech_{n}>::entry("{n}"),' for n in entries]

@@ -35,7 +35,9 @@ struct ohc_ctx {
                                 // mechanism needs the general kernel)
     int grid = 0;  // persistent integrator grid (single-wavefront blocks)
     int cus = 0;         // compute units of the device
+    int quad_per_cu = 0; // resident blocks per CU of the four-cell integrator (0: none)
     int max_per_cu = 0;  // resident integrator blocks per CU the kernel allows
+    int quad_max_per_cu = 0;
     unsigned long long *d_ctl = nullptr;  // [0] queue head, [1..8] stats
     std::vector<void *> stage;            // host-pointer staging buffers
     std::vector<size_t> stage_sz;
@@ -170,8 +172,10 @@ int stats_from_words(ohc_ctx *c, const unsigned long long *words, ohc_stats *st)
 // Integrator parameters that come from the context options (pointers, n and
 // the queue left zero).
 void base_params(const ohc_ctx *c, ohcd::LaneParams &P);
-// Launch the context's integrator kernel (lane or generic) on its stream.
-hipError_t launch_integrator(const ohc_ctx *c, const ohcd::LaneParams &P);
+// Launch the context's integrator kernel (lane or generic) on its stream for
+// the P.n queued cells of a call of n cells: n, not P.n, chooses between kernels,
+// so that slices and listed cells take the same one as the whole call.
+hipError_t launch_integrator(const ohc_ctx *c, const ohcd::LaneParams &P, int64_t n);
 // chemistrySource::solve (mode 0) / solveUpdate (mode 1) over n cells; with a
 // device list of cell indices only those nlist cells are integrated.
 int chem_integrate(ohc_ctx *c, int mode, int64_t n, const double *T, double *Tio,

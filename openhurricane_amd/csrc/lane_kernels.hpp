@@ -1331,7 +1331,16 @@ struct LaneEntry {
     hipError_t (*tfromh)(const ThParams &, hipStream_t);
     const void *integrate_fn;
     hipError_t (*source)(const SourceParams &, hipStream_t);
+    // ImplicitEuler in FP64 with four cells per wavefront (quad_lane.hpp); its
+    // kernel is null where the mechanism does not fit
+    hipError_t (*integrate_quad)(const LaneParams &, int grid, hipStream_t);
+    const void *quad_fn;
 };
+
+template <class M>
+hipError_t launch_quad_lane(const LaneParams &, int grid, hipStream_t);
+template <class M>
+const void *quad_lane_fn();
 
 template <class M>
 struct LaneLaunch {
@@ -1379,7 +1388,8 @@ struct LaneLaunch {
     static LaneEntry entry(const char *name) {
         return LaneEntry{name,    M::HASH, M::THASH, M::NS,
                          &integrate, &eval,  &props,   &tfromh,
-                         (const void *)&ie_lane_kernel<M, 0>, &source};
+                         (const void *)&ie_lane_kernel<M, 0>, &source,
+                         &launch_quad_lane<M>, quad_lane_fn<M>()};
     }
 };
 

@@ -122,7 +122,7 @@ extern "C" int ohc_chem_solve_update_noalloc(ohc_ctx *c, int64_t n, double *T, c
     }
     hipLaunchKernelGGL(noalloc_reset, dim3(1), dim3(64), 0, c->stream, ctl);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, ohci::launch_integrator(c, P));
+    HIPCHK(c, ohci::launch_integrator(c, P, n));
     if (!stats) return OHC_OK;
     unsigned long long h[8];
     HIPCHK(c, hipMemcpyAsync(h, ctl + 1, sizeof(h), hipMemcpyDeviceToHost, c->stream));

@@ -365,19 +365,31 @@ void base_params(const ohc_ctx *c, ohcd::LaneParams &P) {
     P.integrator = o.integrator;
 }
 
-hipError_t launch_integrator(const ohc_ctx *c, const ohcd::LaneParams &P) {
+// Calls of up to this many cells run four cells per wavefront on compiled
+// mechanisms (quad_lane.hpp): beyond, the time is that of the work, which one
+// lane per cell does in a quarter of the instructions.  131,072 H2-air cells take
+// 210 ms here and 264 ms there, 262,144 366 and 275.
+constexpr int64_t kQuadLaneMax = 1 << 17;
+
+// Cells that a wavefront of the integrator holds at a time in a call of n cells.
+static int cells_per_wave(const ohc_ctx *c, int64_t n) {
+    if (c->lane) return c->quad_per_cu > 0 && n <= kQuadLaneMax ? 4 : 64;
+    return ohcd::wave_cells(c->mech.ns + 1, c->opts.integrator, c->opts.precision, n);
+}
+
+hipError_t launch_integrator(const ohc_ctx *c, const ohcd::LaneParams &P, int64_t n) {
     if (P.n <= 0) return hipSuccess;
-    if (c->lane) {
-        const int grid = (int)std::min<int64_t>(c->grid, (P.n + 63) / 64);
-        return c->lane->integrate(P, grid, c->stream);
-    }
+    const int per = cells_per_wave(c, n);
+    const int64_t full = per == 4 ? (int64_t)c->cus * c->quad_per_cu : c->grid;
+    const int grid = (int)std::min<int64_t>(full, (P.n + per - 1) / per);
+    if (c->lane)
+        return per == 4 ? c->lane->integrate_quad(P, grid, c->stream)
+                        : c->lane->integrate(P, grid, c->stream);
     ohcd::WaveParams W;
     W.L = P;
     W.M = c->wm;
     W.exact_dkp = c->opts.jacobian;
-    const int per = ohcd::wave_cells(c->mech.ns + 1, P.integrator);
-    const int grid = (int)std::min<int64_t>(c->grid, (P.n + per - 1) / per);
-    return ohcd::wave_integrate(W, grid, c->stream);
+    return ohcd::wave_integrate(W, per, grid, c->stream);
 }
 
 int stats_from_words(ohc_ctx *c, const unsigned long long *h, ohc_stats *st) {
@@ -494,7 +506,7 @@ int chem_integrate(ohc_ctx *c, int mode, int64_t n, const double *T, double *Tio
     P.stats = c->d_ctl + 1;
     hipLaunchKernelGGL(reset_ctl, dim3(1), dim3(64), 0, c->stream, c->d_ctl);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, launch_integrator(c, P));
+    HIPCHK(c, launch_integrator(c, P, std::max(n, c->sliced_n)));
     if (sched) {
         // next call on these cells: most expensive first
         HIPCHK(c, ohcs::order_by_cost(c->d_cost, c->d_order, c->d_bins, n, c->stream));
@@ -688,10 +700,21 @@ int ohc_ctx_create(const ohc_mech *m, const ohc_opts *opts, int32_t device, ohc_
         hipDeviceProp_t prop;
         HIPCHK(cp, hipGetDeviceProperties(&prop, device));
         int per_cu = 0;
-        const void *fn = c->lane ? c->lane->integrate_fn : ohcd::wave_integrate_fn(c->mech.ns + 1, o.integrator);
+        const void *fn = c->lane ? c->lane->integrate_fn : ohcd::wave_integrate_fn(c->mech.ns + 1, 1);
         HIPCHK(cp, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64, 0));
         c->cus = prop.multiProcessorCount;
         c->max_per_cu = std::max(per_cu, 1);
+        const void *quad = nullptr;
+        if (c->lane) {
+            if (o.integrator == 0 && o.precision == 0) quad = c->lane->quad_fn;
+        } else if (ohcd::wave_cells(c->mech.ns + 1, o.integrator, o.precision, INT64_MAX) == 4) {
+            quad = ohcd::wave_integrate_fn(c->mech.ns + 1, 4);
+        }
+        if (quad) {
+            HIPCHK(cp, hipOccupancyMaxActiveBlocksPerMultiprocessor(&c->quad_per_cu, quad, 64, 0));
+            c->quad_per_cu = c->quad_max_per_cu = std::max(c->quad_per_cu, 1);
+            if (o.waves_per_cu > 0) c->quad_per_cu = std::min(c->quad_per_cu, o.waves_per_cu);
+        }
         if (o.waves_per_cu > 0) per_cu = std::min(per_cu, o.waves_per_cu);
         if (per_cu < 1) per_cu = 1;
         c->grid = prop.multiProcessorCount * per_cu;
@@ -771,13 +794,19 @@ int ohc_ctx_autotune(ohc_ctx *c, int64_t n, const double *T, const double *p, co
                    : chem_integrate(c, 1, n, nullptr, hT.data(), p, rho, nullptr, hY.data(), ldY,
                                     dt, dtFactor, hsub.data(), nullptr, n, nullptr, nullptr, 0);
     };
-    const int keep = c->grid;
+    // the grid of the kernel that a call of n cells takes
+    const bool quad = cells_per_wave(c, n) == 4;
+    auto set_per_cu = [&](int w) {
+        if (quad) c->quad_per_cu = w;
+        else c->grid = c->cus * w;
+    };
+    const int keep = quad ? c->quad_per_cu : c->grid / c->cus;
     int best = 0;
     float best_t = 0.0f;
     // from the most resident blocks down; stop once a size is clearly slower
     // than the best so far (the step time is unimodal in the grid size)
-    for (int w = c->max_per_cu; w >= 1 && !rc; --w) {
-        c->grid = c->cus * w;
+    for (int w = quad ? c->quad_max_per_cu : c->max_per_cu; w >= 1 && !rc; --w) {
+        set_per_cu(w);
         if (dev) {
             if (!ok(hipMemsetAsync(dsub, 0, sv, c->stream), "hipMemsetAsync")) break;
         } else {
@@ -807,10 +836,10 @@ int ohc_ctx_autotune(ohc_ctx *c, int64_t n, const double *T, const double *p, co
     if (dY) (void)hipFree(dY);
     if (dsub) (void)hipFree(dsub);
     if (rc || best == 0) {
-        c->grid = keep;
+        set_per_cu(keep);
         return rc ? rc : fail(c, OHC_ERR_DEVICE, "autotune found no working configuration");
     }
-    c->grid = c->cus * best;
+    set_per_cu(best);
     c->opts.waves_per_cu = best;
     if (waves_per_cu) *waves_per_cu = best;
     if (best_ms) *best_ms = best_t;

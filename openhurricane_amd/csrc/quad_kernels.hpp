@@ -1,17 +1,19 @@
-// quad_kernels.hpp -- generic (run-time mechanism table) integrator for up to
-// 32 species: one wavefront integrates four cells, 16 lanes each.
+// quad_kernels.hpp -- integrator with four cells per wavefront, 16 lanes each,
+// for mechanisms of up to 15 species: on run-time tables (TableSys, here) and on
+// compiled mechanisms (CompiledSys, quad_lane.hpp).
 //
-// Why 16 lanes per cell.  A cell's Newton iteration is one Jacobian
-// evaluation and one dense solve.  gfx950 moves a 64-bit value from one lane
-// to the 16 lanes of its row in a single vector instruction
-// (v_mov_b64_dpp row_newbcast), so a matrix whose rows are spread over one
-// row of lanes (row i in lane i % 16, slot i / 16) is eliminated with one move
-// per pivot-row element and one FMA per slot, all 64 lanes busy with four
-// cells: 1.7k vector instructions per four 32-species solves, where one
-// wavefront per cell needs a pair of v_readlane per element and leaves half
-// its lanes idle (3k per solve).  Reactions are evaluated 16 at a time in each
-// group, so the 64-lane table chunks are read in quarters and a quarter mostly
-// holds one kind of reaction.
+// Why 16 lanes per cell.  A cell's Newton iteration is one Jacobian evaluation
+// and one dense solve, a serial chain whose length is all that a call of few
+// cells sees.  gfx950 moves a 64-bit value from one lane to the 16 lanes of its
+// row in a single vector instruction (v_mov_b64_dpp row_newbcast), so a matrix
+// with row i in lane i of the group is eliminated with one move and one FMA per
+// pivot-row element, for four cells at once; one wavefront per cell needs a pair
+// of v_readlane per element and leaves 52 lanes idle, one lane per cell runs
+// every element of the matrix one after the other.  Reactions are evaluated 16
+// at a time in each group.  Above 16 rows a lane holds two rows and the LDS holds
+// two wavefronts per SIMD at most: at 33 rows that measured no better than one
+// wavefront per cell (440 against 445 ms on 524,288 cells), so those sizes stay
+// there.
 //
 // The elimination order is fixed (lane numbers of DPP broadcasts are
 // immediates): Gauss-Jordan without row exchanges on the species block of
@@ -25,6 +27,12 @@
 // of a lane: each group holds one cell, takes the wavefront-wide evaluation and
 // solve together with the other three, and refills from the work queue by
 // itself.  References as in wave_kernels.hpp.
+//
+// Measured, one ImplicitEuler flow step of the H2-air tables (9 species, 19
+// reactions), one wavefront per cell -> four cells per wavefront: 65,536 cells
+// 445 -> 278 ms, 32,768 289 -> 240, 8,192 221 -> 209, 4,096 190 -> 187, but 2,048
+// 168 -> 187 and 64 140 -> 151: few cells leave the chip idle either way, and the
+// 64-lane reaction loop of one cell is the shorter chain (kQuadTableMin).
 #pragma once
 
 #include "wave_kernels.hpp"
@@ -33,6 +41,8 @@ namespace ohcd {
 
 // largest ODE size (species + 1) of the four-cell kernels
 constexpr int kQuadMaxN = 16;
+// smallest call that takes them on a run-time mechanism table
+constexpr int64_t kQuadTableMin = 4096;
 
 template <int N>
 struct QuadShape {
@@ -90,6 +100,31 @@ __device__ __forceinline__ double rcp_raw(double x) {
     return fma(fma(-x, r, 1.0), r, r);
 }
 
+// ln x to a few 1e-16 of max(1, |ln x|), x held to [1e-290, 1e290]: mantissa m in
+// [sqrt(1/2), sqrt(2)), s = (m - 1) / (m + 1), the series of 2 artanh(s); half the
+// library logarithm's dependent chain and no branch.
+__device__ __forceinline__ double log_pos(double x) {
+    x = fmin(fmax(x, 1.0e-290), 1.0e290);
+    double m = __builtin_amdgcn_frexp_mant(x);
+    int e = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    e -= low ? 1 : 0;
+    const double s = (m - 1.0) * rcp_raw(m + 1.0), z = s * s, y = z * z;
+    // even and odd powers apart: two shorter chains
+    double p = 2.0 / 21.0, q = 2.0 / 19.0;
+    p = fma(p, y, 2.0 / 17.0);
+    q = fma(q, y, 2.0 / 15.0);
+    p = fma(p, y, 2.0 / 13.0);
+    q = fma(q, y, 2.0 / 11.0);
+    p = fma(p, y, 2.0 / 9.0);
+    q = fma(q, y, 2.0 / 7.0);
+    p = fma(p, y, 2.0 / 5.0);
+    q = fma(q, y, 2.0 / 3.0);
+    p = fma(p, y, 2.0);
+    return fma((double)e, 0.69314718055994530942, s * fma(q, z, p));
+}
+
 // What the Newton system needs of one evaluation, besides J in LDS.
 template <int S>
 struct QuadF {
@@ -100,7 +135,7 @@ struct QuadF {
 };
 
 // dy/dt and J of each group's cell at (y, T): species c + 16 s in slot s.
-template <int N, int FLOW, class F>
+template <int N, int FLOW>
 __device__ __forceinline__ void quad_eval(const WMech &M, QuadLDS<N> &L,
                                           const double (&y)[QuadShape<N>::S], double T, int exact,
                                           QuadF<QuadShape<N>::S> &o) {
@@ -116,7 +151,7 @@ __device__ __forceinline__ void quad_eval(const WMech &M, QuadLDS<N> &L,
         o.H[s] = o.C[s] = dCp[s] = 0.0;
         if (k < ns) {
             double G, dG, Cp, H;
-            wthermo<F>(M, k, tf, G, dG, Cp, H, dCp[s]);
+            wthermo(M, k, tf, G, dG, Cp, H, dCp[s]);
             L.c[g][k] = fmax(y[s], 0.0);
             L.G[g][k] = G;
             L.dG[g][k] = dG;
@@ -139,7 +174,7 @@ __device__ __forceinline__ void quad_eval(const WMech &M, QuadLDS<N> &L,
         WRxn x;
         x.nf = x.nb = 0;
         if (r < M.nr) {
-            wreaction<true, F>(M, base >> 6, tl, tf, L.c[g], L.G[g], L.dG[g], exact, x);
+            wreaction<true>(M, base >> 6, tl, tf, L.c[g], L.G[g], L.dG[g], exact, x);
 #pragma unroll
             for (int side = 0; side < 2; ++side) {
 #pragma unroll
@@ -280,31 +315,31 @@ __device__ __noinline__ void quad_solve_pivoted(QuadLDS<N> &L, int gg, double h,
 // (I - h J) x = b for the four groups' cells: species rows b, x by slot, the
 // temperature row bT, xT in every lane of the group.  act: groups whose
 // solution is used (the others solve whatever their LDS holds).
-template <int N>
-__device__ __forceinline__ void quad_solve(QuadLDS<N> &L, double h,
+// jac(s, j): J of row slot s, column j (NS: d/dT), a compile-time index.
+// to_lds(): puts the group's J into L.J for the pivoted solve.
+template <int N, class JAC, class PUT>
+__device__ __forceinline__ void quad_solve(QuadLDS<N> &L, JAC &&jac, PUT &&to_lds, double h,
                                            const double (&b)[QuadShape<N>::S], double bT,
                                            const QuadF<QuadShape<N>::S> &o, bool act,
                                            double (&x)[QuadShape<N>::S], double &xT) {
     using Q = QuadShape<N>;
     constexpr int S = Q::S, NS = Q::NS;
     const int lane = threadIdx.x, c = lane & 15, g = lane >> 4;
-    const double *Jr[S];
     double a[S][NS], bb[S], u[S], u0[S], jT[S], rpv[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int i = c + 16 * s;
         const bool ok = i < NS;
-        Jr[s] = L.J + g * Q::CST + (ok ? i : 0) * Q::JS;
         sfor<0, NS>([&](auto j) {
             // -h J, then + 1 on the diagonal: two roundings, as the reference
             // forms I - h J (ImplicitEuler.cpp:186-193)
 #pragma clang fp contract(off)
-            const double v = NS % 16 == 0 || ok ? -h * Jr[s][j] : 0.0;
+            const double v = NS % 16 == 0 || ok ? -h * jac(s, j) : 0.0;
             const bool dj = s == j / 16 && __builtin_amdgcn_inverse_ballot_w64(
                                                0x0001000100010001ull << (j % 16));
             a[s][j] = s == j / 16 ? v + (dj ? 1.0 : 0.0) : v;
         });
-        jT[s] = NS % 16 == 0 || ok ? Jr[s][NS] : 0.0;
+        jT[s] = NS % 16 == 0 || ok ? jac(s, std::integral_constant<int, NS>{}) : 0.0;
         bb[s] = b[s];
         u0[s] = u[s] = -h * jT[s];
         rpv[s] = 0.0;
@@ -365,7 +400,7 @@ __device__ __forceinline__ void quad_solve(QuadLDS<N> &L, double h,
         const double t = rbcast<j % 16>(x[j / 16]);
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            const double v = Jr[s][j];
+            const double v = jac(s, j);
             jx[s] = fma(v, t, jx[s]);
             ax[s] = fma(fabs(v), fabs(t), ax[s]);
         }
@@ -395,6 +430,7 @@ __device__ __forceinline__ void quad_solve(QuadLDS<N> &L, double h,
     unsigned long long rm = __builtin_amdgcn_ballot_w64(redo);
     if (rm) {
         if (redo) {
+            to_lds();
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 const int i = c + 16 * s;
@@ -425,23 +461,58 @@ __device__ __forceinline__ void quad_solve(QuadLDS<N> &L, double h,
     }
 }
 
+// The system of a run-time mechanism table.
+template <int N, int FLOW>
+struct TableSys {
+    using Params = WaveParams;
+    static constexpr int kN = N, S = QuadShape<N>::S, kWavesPerSimd = 2;
+    using Lds = QuadLDS<N>;
+    int ns;
+    double W[S];
+    static __device__ __forceinline__ const LaneParams &lane(const Params &p) { return p.L; }
+    __device__ __forceinline__ void init(const Params &p, Lds &) {
+        ns = p.M.ns;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int k = (threadIdx.x & 15) + 16 * s;
+            W[s] = k < ns ? p.M.sp[SP_W * 64 + k] : 1.0;
+        }
+    }
+    __device__ __forceinline__ void step(const Params &p, Lds &L, const double (&yk)[S], double ykT,
+                                         const double (&y0)[S], double y0T, double h, bool act,
+                                         QuadF<S> &o, double (&x)[S], double &xT) {
+        using Q = QuadShape<N>;
+        const int c = threadIdx.x & 15, g = threadIdx.x >> 4;
+        quad_eval<N, FLOW>(p.M, L, yk, ykT, p.exact_dkp, o);
+        double b[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) b[s] = c + 16 * s < ns ? -yk[s] + y0[s] + h * o.w[s] : 0.0;
+        const double bT = -ykT + y0T + h * -o.dT;
+        const double *J = L.J + g * Q::CST;
+        auto jac = [&](int s, auto j) __attribute__((always_inline)) {
+            const int i = c + 16 * s;
+            return J[(i < Q::NS ? i : 0) * Q::JS + j];
+        };
+        quad_solve<N>(L, jac, [] {}, h, b, bT, o, act, x, xT);
+    }
+};
+
 // Persistent integrator: ImplicitEuler (ImplicitEuler.cpp:40-342) under
-// chemistrySource::solve / solveUpdate, four cells per wavefront.  F = float:
-// the split-precision mode.
-template <int N, int FLOW, class F = double>
-__global__ __launch_bounds__(64, (N <= 24 ? 2 : 1)) void ie_quad_kernel(const WaveParams WP) {
-    using Q = QuadShape<N>;
-    constexpr int S = Q::S;
-    const LaneParams &P = WP.L;
-    const WMech &M = WP.M;
-    const int lane = threadIdx.x, c = lane & 15, ns = M.ns;
-    __shared__ QuadLDS<N> L;
+// chemistrySource::solve / solveUpdate, four cells per wavefront.
+template <class SYS>
+__global__ __launch_bounds__(64, SYS::kWavesPerSimd) void ie_quad_kernel(
+    const typename SYS::Params WP) {
+    constexpr int S = SYS::S;
+    const LaneParams &P = SYS::lane(WP);
+    const int lane = threadIdx.x, c = lane & 15;
+    __shared__ typename SYS::Lds L;
+    SYS sys;
+    sys.init(WP, L);
+    const int ns = sys.ns;
+    const double(&W)[S] = sys.W;
     enum { PQ_NEED, PQ_NEWTON, PQ_ERR0, PQ_DONE };
     int phase = PQ_NEED;
     const double errg = pow(P.maxsc / P.safe, -1.0 / P.alpha);
-    double W[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) W[s] = c + 16 * s < ns ? M.sp[SP_W * 64 + c + 16 * s] : 1.0;
     // the group's cell: step start y0, previous step start yl, Newton iterate
     // yk (species by slot, temperature in every lane), and the controller
     double y0[S], yl[S], yk[S], y0T = 1000.0, ylT = 1000.0, ykT = 1000.0;
@@ -563,27 +634,13 @@ __global__ __launch_bounds__(64, (N <= 24 ? 2 : 1)) void ie_quad_kernel(const Wa
         citer = 0;
         start_ode();
     };
-    // ImplicitEuler::maxIncrement of the error vector e, eT
-    auto max_increment = [&](const double(&e)[S], double eT) __attribute__((always_inline)) {
-        double m = fabs(eT) * frcp(P.atol_inc + P.rtol_inc * fmax(fabs(y0T), fabs(ykT)));
-        bool nan_y = isnan(ykT);
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-            if (c + 16 * s < ns) {
-                nan_y = nan_y || isnan(yk[s]);
-                const double tol = P.atol_inc + P.rtol_inc * fmax(fabs(y0[s]), fabs(yk[s]));
-                m = fmax(m, fabs(e[s]) * frcp(tol));
-            }
-        m = gmax(m);
-        return gany(nan_y) ? 1.5 : m;
-    };
     // checkNewY and the step-size control of adaptiveSolve, then the loops of
     // ImplicitEuler::solve and chemistrySource::solve
     auto attempt_done = [&](double error) __attribute__((always_inline)) {
         enum { A_RETRY, A_FAIL, A_NEXT, A_ODE_END };
         int action;
         // error^-alpha, wherever a branch below needs it
-        const double pw = exp(-P.alpha * log(error));
+        const double pw = exp(-P.alpha * log_pos(error));
         const bool ok = !((ykT - y0T) > P.Talpha * y0T);
         if (!ok) dtl *= P.Tbeta;
         if (!ok && chk < 100) {
@@ -651,71 +708,67 @@ __global__ __launch_bounds__(64, (N <= 24 ? 2 : 1)) void ie_quad_kernel(const Wa
         if (!__any(phase != PQ_DONE)) break;
         // ---- f and J at the Newton iterates, and the Newton systems ----
         QuadF<S> o;
-        quad_eval<N, FLOW, F>(M, L, yk, ykT, WP.exact_dkp, o);
-        double x[S], xT, b[S], bT;
+        double x[S], xT;
+        sys.step(WP, L, yk, ykT, y0, y0T, dtl, phase == PQ_NEWTON, o, x, xT);
+        // ---- Newton update, its norm and the error estimate: straight-line for
+        // all groups, so that the two maxima run side by side ----
+        const bool newton = phase == PQ_NEWTON, err0 = phase == PQ_ERR0;
+        bool bad_x = bad(xT);
 #pragma unroll
-        for (int s = 0; s < S; ++s) b[s] = c + 16 * s < ns ? -yk[s] + y0[s] + dtl * o.w[s] : 0.0;
-        bT = -ykT + y0T + dtl * -o.dT;
-        quad_solve<N>(L, dtl, b, bT, o, phase == PQ_NEWTON, x, xT);
+        for (int s = 0; s < S; ++s) bad_x = bad_x || bad(x[s]);
+        bad_x = gany(bad_x);
+        const bool upd = newton && !bad_x;
+        ykT += upd ? xT : 0.0;
+        double m1 = fabs(xT) * frcp(P.atol + P.rtol * fabs(ykT));
+        // first step: y - y0 - dt f(y) (ImplicitEuler.cpp:111-120); later the
+        // second-difference LTE (ImplicitEuler.cpp:122-139)
+        const double e1 = lts0 * frcp(lts0 + lts1), e2 = e1 * lts0 * frcp(lts1);
+        const double eT = err0 ? ykT - y0T + dtl * o.dT : e1 * (ykT - y0T) - e2 * (y0T - ylT);
+        double m2 = fabs(eT) * frcp(P.atol_inc + P.rtol_inc * fmax(fabs(y0T), fabs(ykT)));
+        bool nan_y = isnan(ykT);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            yk[s] += upd ? x[s] : 0.0;
+            const double e = err0 ? yk[s] - y0[s] - dtl * o.w[s]
+                                  : e1 * (yk[s] - y0[s]) - e2 * (y0[s] - yl[s]);
+            if (c + 16 * s < ns) {
+                m1 = fmax(m1, fabs(x[s]) * frcp(P.atol + P.rtol * fabs(yk[s])));
+                m2 = fmax(m2, fabs(e) * frcp(P.atol_inc + P.rtol_inc * fmax(fabs(y0[s]), fabs(yk[s]))));
+                nan_y = nan_y || isnan(yk[s]);
+            }
+        }
+        m1 = gmax(m1);
+        m2 = gmax(m2);
+        if (gany(nan_y)) m2 = 1.5;  // ImplicitEuler::maxIncrement
         // ---- group-local transitions ----
         bool have = false;
         double aerr = 0.0;
-        if (phase == PQ_ERR0) {
-            // first step: e = y - y0 - dt f(y) (ImplicitEuler.cpp:111-120)
+        if (err0) {
             ++c_rhs;
-            double e[S];
-#pragma unroll
-            for (int s = 0; s < S; ++s) e[s] = yk[s] - y0[s] - dtl * o.w[s];
-            aerr = max_increment(e, ykT - y0T - dtl * -o.dT);
             have = true;
-        } else if (phase == PQ_NEWTON) {
+            aerr = m2;
+        } else if (newton) {
             // NewtonIteration after the solve (ImplicitEuler.cpp:200-249)
             ++c_newt;
             ++citer;
-            bool bad_x = bad(xT);
-#pragma unroll
-            for (int s = 0; s < S; ++s) bad_x = bad_x || bad(x[s]);
-            if (gany(bad_x)) {
+            if (bad_x || (ncount > 5 && m1 > 2.0 * fmax(lastErr, kTiny))) {
                 have = true;
                 aerr = 1000.0;
             } else {
-                ykT += xT;
-                double maxErr = fabs(xT) * frcp(P.atol + P.rtol * fabs(ykT));
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    yk[s] += x[s];
-                    if (c + 16 * s < ns)
-                        maxErr = fmax(maxErr, fabs(x[s]) * frcp(P.atol + P.rtol * fabs(yk[s])));
-                }
-                maxErr = gmax(maxErr);
-                if (ncount > 5 && (maxErr / fmax(lastErr, kTiny)) > 2) {
+                lastErr = m1;
+                ++ncount;
+                if (isnan(m1)) {
                     have = true;
                     aerr = 1000.0;
-                } else {
-                    lastErr = maxErr;
-                    ++ncount;
-                    if (isnan(maxErr)) {
-                        have = true;
-                        aerr = 1000.0;
-                    } else if (ncount > 1000) {
-                        have = true;
-                        aerr = maxErr;
-                    } else if (maxErr > 1.0) {
-                        // iterate again at the new yk
-                    } else if (nstep == 0) {
+                } else if (ncount > 1000) {
+                    have = true;
+                    aerr = m1;
+                } else if (m1 <= 1.0) {
+                    if (nstep == 0) {
                         phase = PQ_ERR0;
                     } else {
-                        // second-difference LTE (ImplicitEuler.cpp:122-139)
-                        const double f1 = 2.0 / (lts0 * (lts0 + lts1));
-                        const double f2 = 2.0 / (lts1 * (lts0 + lts1));
-                        const double LTEF = lts0 * lts0 * 0.5;
-                        double e[S];
-#pragma unroll
-                        for (int s = 0; s < S; ++s)
-                            e[s] = (f1 * (yk[s] - y0[s]) - f2 * (y0[s] - yl[s])) * LTEF;
-                        aerr = max_increment(
-                            e, (f1 * (ykT - y0T) - f2 * (y0T - ylT)) * LTEF);
                         have = true;
+                        aerr = m2;
                     }
                 }
             }

@@ -9,7 +9,7 @@
 namespace ohcd {
 
 #define OHC_WAVE_DECL(n)                                                           \
-    hipError_t wave_integrate_##n(const WaveParams &, int, hipStream_t);             \
+    hipError_t wave_integrate_##n(const WaveParams &, int, int, hipStream_t);             \
     hipError_t wave_eval_##n(const EvalParams &, const WMech &, int, hipStream_t);  \
     hipError_t wave_source_##n(const SourceParams &, const WMech &, hipStream_t);    \
     hipError_t wave_kim_##n(const KimParams &, const WMech &, int, hipStream_t);     \
@@ -28,7 +28,7 @@ OHC_WAVE_DECL(64)
 namespace {
 struct Entry {
     int N;
-    hipError_t (*integrate)(const WaveParams &, int, hipStream_t);
+    hipError_t (*integrate)(const WaveParams &, int, int, hipStream_t);
     hipError_t (*eval)(const EvalParams &, const WMech &, int, hipStream_t);
     hipError_t (*source)(const SourceParams &, const WMech &, hipStream_t);
     hipError_t (*kim)(const KimParams &, const WMech &, int, hipStream_t);
@@ -55,9 +55,9 @@ int wave_size(int n) {
     return e ? e->N : -1;
 }
 
-hipError_t wave_integrate(const WaveParams &p, int grid, hipStream_t s) {
+hipError_t wave_integrate(const WaveParams &p, int cells, int grid, hipStream_t s) {
     const Entry *e = pick(p.M.ns + 1);
-    return e ? e->integrate(p, grid, s) : hipErrorInvalidValue;
+    return e ? e->integrate(p, cells, grid, s) : hipErrorInvalidValue;
 }
 
 hipError_t wave_eval(const EvalParams &p, const WMech &m, int exact, hipStream_t s) {
@@ -203,14 +203,14 @@ hipError_t wave_props(const PropParams &p, const WMech &m, hipStream_t s) {
     return hipGetLastError();
 }
 
-const void *wave_integrate_fn(int n, int integrator) {
+const void *wave_integrate_fn(int n, int cells) {
     const Entry *e = pick(n);
-    return e ? e->fn(integrator) : nullptr;
+    return e ? e->fn(cells) : nullptr;
 }
 
-int wave_cells(int n, int integrator) {
+int wave_cells(int n, int integrator, int prec, int64_t ncells) {
     const Entry *e = pick(n);
-    return e && e->N <= kQuadMaxN && integrator == 0 ? 4 : 1;
+    return e && e->N <= kQuadMaxN && integrator == 0 && prec == 0 && ncells >= kQuadTableMin ? 4 : 1;
 }
 
 }  // namespace ohcd

@@ -12,17 +12,20 @@
 
 namespace ohcd {
 
-// ImplicitEuler: four cells per wavefront up to kQuadMaxN unknowns, one above
-// (a lane would hold more rows of the system than its registers).
-template <int N, int FLOW, class F>
-static void launch_ie(const WaveParams &p, int grid, hipStream_t s) {
-    if constexpr (N <= kQuadMaxN)
-        hipLaunchKernelGGL((ie_quad_kernel<N, FLOW, F>), dim3(grid), dim3(64), 0, s, p);
-    else
-        hipLaunchKernelGGL((ie_wave_kernel<N, FLOW, 0, F>), dim3(grid), dim3(64), 0, s, p);
+// ImplicitEuler, one or four (N <= kQuadMaxN) cells per wavefront
+template <int N, int FLOW>
+static void launch_ie(const WaveParams &p, int cells, int grid, hipStream_t s) {
+    if constexpr (N <= kQuadMaxN) {
+        if (cells == 4) {
+            hipLaunchKernelGGL((ie_quad_kernel<TableSys<N, FLOW>>), dim3(grid), dim3(64), 0, s, p);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((ie_wave_kernel<N, FLOW, 0>), dim3(grid), dim3(64), 0, s, p);
 }
 
-hipError_t OHC_CAT(wave_integrate_, OHC_WAVE_N)(const WaveParams &p, int grid, hipStream_t s) {
+hipError_t OHC_CAT(wave_integrate_, OHC_WAVE_N)(const WaveParams &p, int cells, int grid,
+                                                 hipStream_t s) {
     constexpr int N = OHC_WAVE_N;
     if (p.L.integrator == 4) {
         if (p.L.flow == 0) hipLaunchKernelGGL((mts_wave_kernel<N, 0>), dim3(grid), dim3(64), 0, s, p);
@@ -34,12 +37,12 @@ hipError_t OHC_CAT(wave_integrate_, OHC_WAVE_N)(const WaveParams &p, int grid, h
         if (p.L.flow == 0) hipLaunchKernelGGL((ie_wave_kernel<N, 0, 2>), dim3(grid), dim3(64), 0, s, p);
         else hipLaunchKernelGGL((ie_wave_kernel<N, 1, 2>), dim3(grid), dim3(64), 0, s, p);
     } else if (p.L.prec == 1) {
-        if (p.L.flow == 0) launch_ie<N, 0, float>(p, grid, s);
-        else launch_ie<N, 1, float>(p, grid, s);
+        if (p.L.flow == 0) hipLaunchKernelGGL((ie_wave_kernel<N, 0, 0, float>), dim3(grid), dim3(64), 0, s, p);
+        else hipLaunchKernelGGL((ie_wave_kernel<N, 1, 0, float>), dim3(grid), dim3(64), 0, s, p);
     } else if (p.L.flow == 0) {
-        launch_ie<N, 0, double>(p, grid, s);
+        launch_ie<N, 0>(p, cells, grid, s);
     } else {
-        launch_ie<N, 1, double>(p, grid, s);
+        launch_ie<N, 1>(p, cells, grid, s);
     }
     return hipGetLastError();
 }
@@ -78,14 +81,12 @@ hipError_t OHC_CAT(wave_lu_, OHC_WAVE_N)(const LuParams &p, hipStream_t s) {
     return hipGetLastError();
 }
 
-const void *OHC_CAT(wave_fn_, OHC_WAVE_N)(int integrator) {
+const void *OHC_CAT(wave_fn_, OHC_WAVE_N)(int cells) {
     constexpr int N = OHC_WAVE_N;
     if constexpr (N <= kQuadMaxN) {
-        if (integrator == 0) return (const void *)&ie_quad_kernel<N, 0>;
-        return (const void *)&ie_wave_kernel<N, 0, 2>;
-    } else {
-        return (const void *)&ie_wave_kernel<N, 0>;
+        if (cells == 4) return (const void *)&ie_quad_kernel<TableSys<N, 0>>;
     }
+    return (const void *)&ie_wave_kernel<N, 0>;
 }
 
 }  // namespace ohcd
