@@ -249,6 +249,95 @@ __device__ __forceinline__ void species_CH(double T, double &Cp, double &H, doub
     species_CH<M, k>(Coef<M, k>(T), T, Cp, H, dCp);
 }
 
+// The thermo polynomials of a compiled mechanism per mole, in LDS, for kernels
+// of one cell per lane: a wavefront whose cells lie on both sides of Tcommon reads
+// each lane's coefficients there, where compile-time constants cost two moves and
+// two selects each (1,050 of 1,700 vector instructions of the thermo of 9
+// species).  Pairs of coefficients, low and high range side by side, so that a
+// lane's 16-byte read never shares a bank with the other range's.
+template <class M>
+struct ThermoTab {
+    enum { T_S, T_G = 6, T_C = 12, T_H = 17, T_D = 22, T_N = 26 };  // T_S..T_G: G; T_C..T_D: Cp, H
+    // 4 KB at 16 species: four wavefronts per CU still fit
+    static constexpr bool kFits = M::NS <= 16;
+    static constexpr int kSize = kFits ? M::NS * T_N * 2 : 2;
+    double v[kSize];
+};
+template <class M>
+constexpr ThermoTab<M> thermo_tab() {
+    ThermoTab<M> t{};
+    using Q = ThermoTab<M>;
+    if constexpr (Q::kFits) {
+        for (int k = 0; k < M::NS; ++k)
+            for (int hi = 0; hi < 2; ++hi) {
+                const auto &a = hi ? M::ahi[k] : M::alo[k];
+                const auto &h = hi ? M::hhi[k] : M::hlo[k];
+                const auto &s = hi ? M::shi[k] : M::slo[k];
+                const auto &g = hi ? M::ghi[k] : M::glo[k];
+                const double c[Q::T_N] = {s[0],  s[1],  s[2],  a[1], a[0], a[6], -g[0], -g[1], -g[2],
+                                          -g[3], a[5],  0.0,   a[4], a[3], a[2], a[1],  a[0],  h[0],
+                                          h[1],  h[2],  h[3],  a[5], 4.0 * a[4], 3.0 * a[3], 2.0 * a[2], 0.0};
+                for (int i = 0; i < Q::T_N; ++i)
+                    t.v[k * Q::T_N * 2 + i / 2 * 4 + hi * 2 + i % 2] = c[i] * M::W[k];
+            }
+    }
+    return t;
+}
+template <class M>
+__device__ constexpr ThermoTab<M> kThermoTab = thermo_tab<M>();
+
+// N2 pairs of coefficients of species k from pair P0 on
+template <class M, int k, int P0, int N2>
+__device__ __forceinline__ void thermo_pairs(const double *tab, double T, double (&c)[2 * N2]) {
+    const double *p = tab + (T < M::Tcommon[k] ? 0 : 2) + k * ThermoTab<M>::T_N * 2 + P0 * 4;
+#pragma unroll
+    for (int i = 0; i < N2; ++i) {
+        const double2 v = *(const double2 *)(p + 4 * i);
+        c[2 * i] = v.x;
+        c[2 * i + 1] = v.y;
+    }
+}
+
+// species_G on the table; OUT: some lane is outside the fits (a lane inside gets
+// the same bits either way).  Inside, cp0 and T ds0/dT are the same polynomial.
+template <class M, int k, bool OUT>
+__device__ __forceinline__ void species_G_tab(const double *tab, double T, double lnT, double &G,
+                                              double &dG) {
+    double c[12];
+    thermo_pairs<M, k, 0, 6>(tab, T, c);
+    const double s0 = fma(fma(fma(fma(c[0], T, c[1]), T, c[2]), T, c[3]), T, fma(c[4], lnT, c[5]));
+    const double g0 = fma(fma(fma(c[6], T, c[7]), T, c[8]), T, c[9]);
+    G = fma(fma(g0, T, fma(c[4], 1.0 - lnT, -c[5])), T, c[10]);
+    dG = -s0;
+    if constexpr (OUT) {
+        const double Tl = M::Tlow[k], Th = M::Thigh[k];
+        if (T < Tl || T > Th) {
+            const double Tx = T < Tl ? Tl : Th;
+            double a[6];
+            thermo_pairs<M, k, ThermoTab<M>::T_C / 2, 3>(tab, T, a);
+            dG += fma(fma(fma(fma(a[0], Tx, a[1]), Tx, a[2]), Tx, a[3]), Tx, a[4]) -
+                  fma(fma(fma(fma(a[0], T, a[1]), T, a[2]), T, a[3]), T, a[4]);
+        }
+    }
+}
+
+// species_CH on the table
+template <class M, int k, bool OUT>
+__device__ __forceinline__ void species_CH_tab(const double *tab, double T, double &Cp, double &H,
+                                               double &dCp) {
+    double c[14];
+    thermo_pairs<M, k, ThermoTab<M>::T_C / 2, 7>(tab, T, c);
+    double Tx = T;
+    if constexpr (OUT) {
+        const double Tl = M::Tlow[k], Th = M::Thigh[k];
+        Tx = T < Tl ? Tl : (T > Th ? Th : T);
+    }
+    Cp = fma(fma(fma(fma(c[0], Tx, c[1]), Tx, c[2]), Tx, c[3]), Tx, c[4]);
+    H = fma(fma(fma(fma(fma(c[5], Tx, c[6]), Tx, c[7]), Tx, c[8]), Tx, c[4]), Tx, c[9]);
+    if constexpr (OUT) H = Tx != T ? fma(Cp, T - Tx, H) : H;
+    dCp = fma(fma(fma(c[10], T, c[11]), T, c[12]), T, c[3]);
+}
+
 // species_G evaluated in FP32 (the split-precision mode's Gibbs terms).
 template <class M, int k, int R = -1>
 __device__ __forceinline__ void species_G32(double Td, float lnT, float invTm, double &G,
@@ -596,23 +685,29 @@ __device__ __forceinline__ FallOff<M, r> falloff(const TFac &tf, double Mtb) {
 // net rates, Jacobian, temperature equation) in FP64.
 // UNI: when every lane of the wavefront is above every Tcommon, evaluate the
 // thermo with the high coefficient sets as constants (else per-lane selects).
+// tab: the thermo coefficients in LDS (ThermoTab), or null.
 // MA: mass-action Jacobian only -- the third-body and fall-off q dln(gamma)/dc
 // terms are left out, so that J[k][k] is reactionTable::dWdciAllSpecies's
 // diagonal (the MTS time scales).
 template <class M, bool WITH_J, int FLOW, class F = double, bool UNI = false, bool MA = false>
 __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
                                         double (&f)[M::NS + 1],
-                                        double (&J)[M::NS + 1][M::NS + 1], bool exact = false) {
+                                        double (&J)[M::NS + 1][M::NS + 1], bool exact = false,
+                                        const double *tab = nullptr) {
     constexpr int NS = M::NS, N = NS + 1;
     constexpr bool fp32 = std::is_same_v<F, float>;
+    constexpr bool TAB = UNI && !fp32 && ThermoTab<M>::kFits;
     const double T = y[NS];
     const TFac tf = tfac(T);
-    const bool hi = UNI && wave_all_high<M>(T);
+    const bool hi = UNI && !TAB && wave_all_high<M>(T);
+    const bool out = TAB && __any(T < tlow_max<M>() || T > thigh_min<M>());
     Thermo<M> th;  // G / dG now; Cp / H / dCp after the reaction loop
     auto gibbs = [&](auto Rc) {
         constexpr int R = decltype(Rc)::value;
         sfor<0, NS>([&](auto k) {
-            if constexpr (fp32)
+            if constexpr (TAB)
+                species_G_tab<M, k, R != 0>(tab, T, tf.lnT, th.G[k], th.dG[k]);
+            else if constexpr (fp32)
                 species_G32<M, k, R>(T, (float)tf.lnT, (float)tf.invTm, th.G[k], th.dG[k]);
             else
                 species_G<M, k>(Coef<M, k, R>(T), T, tf.lnT, tf.invTm, th.G[k], th.dG[k]);
@@ -624,7 +719,10 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
             }
         });
     };
-    if (hi) gibbs(std::integral_constant<int, 1>{});
+    if constexpr (TAB) {
+        if (out) gibbs(std::integral_constant<int, 1>{});
+        else gibbs(std::integral_constant<int, 0>{});
+    } else if (hi) gibbs(std::integral_constant<int, 1>{});
     else gibbs(std::integral_constant<int, -1>{});
     double ci[NS];
     sfor<0, NS>([&](auto k) { ci[k] = fmax(y[k], 0.0); });
@@ -777,10 +875,14 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
     auto cph = [&](auto Rc) {
         constexpr int R = decltype(Rc)::value;
         sfor<0, NS>([&](auto k) {
-            species_CH<M, k>(Coef<M, k, R>(T), T, th.Cp[k], th.H[k], th.dCp[k]);
+            if constexpr (TAB) species_CH_tab<M, k, R != 0>(tab, T, th.Cp[k], th.H[k], th.dCp[k]);
+            else species_CH<M, k>(Coef<M, k, R>(T), T, th.Cp[k], th.H[k], th.dCp[k]);
         });
     };
-    if (hi) cph(std::integral_constant<int, 1>{});
+    if constexpr (TAB) {
+        if (out) cph(std::integral_constant<int, 1>{});
+        else cph(std::integral_constant<int, 0>{});
+    } else if (hi) cph(std::integral_constant<int, 1>{});
     else cph(std::integral_constant<int, -1>{});
     double Hx[NS], Cx[NS];
     if constexpr (FLOW == 0) {
@@ -817,71 +919,58 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
     }
 }
 
-// In-place Doolittle LU with partial pivoting of A (registers) applied to b
-// at the same time (the reference's recorded row swaps replayed on b give the
-// same sequence), then forward/back substitution: b <- A^-1 b.
-// Row swaps are done with selects and skipped when no lane of the wavefront
-// needs them.
+// b <- A^-1 b by Gaussian elimination in registers, right-looking (every update
+// is one independent FMA).  A row moves up only where the pivot is below a tenth
+// of a later species' entry in its column: the temperature row (last) has other
+// units, so that comparing it with the species rows says nothing, and it is
+// eliminated last, unless no species row is left with a nonzero entry.  Row swaps
+// are done with selects and skipped when no lane of the wavefront needs them.
+// Exchanging for every larger entry (the temperature row's among them) cost the
+// integrator of 1,048,576 H2-air cells 239 ms a step; with a species row's tenth
+// 232, with the thermo table and this form 203.
 template <int N>
 __device__ __forceinline__ void lu_solve(double (&A)[N][N], double (&b)[N]) {
     double dinv[N];
     sfor<0, N>([&](auto kk) {
         constexpr int k = kk;
-        double s[N];
-        sfor<k, N>([&](auto i) {
-            double sum = 0.0;
-            sfor<0, k>([&](auto t) { sum += A[i][t] * A[t][k]; });
-            s[i] = A[i][k] - sum;
-        });
-        // a row swap is needed where some |s_i| (i > k) exceeds |s_k|; only
-        // then is the pivot row located (the first such maximum, as in the
-        // sequential search)
-        double mo = 0.0;
-        sfor<k + 1, N>([&](auto i) { mo = fmax(mo, fabs(s[i])); });
-        if (__any(mo > fabs(s[k]))) {
-            int ik = k;
-            double maxs = s[k];
-            sfor<k + 1, N>([&](auto i) {
-                const bool g = fabs(s[i]) > fabs(maxs);
-                ik = g ? (int)i : ik;
-                maxs = g ? s[i] : maxs;
-            });
-            sfor<k + 1, N>([&](auto i) {
-                const bool sw = (ik == (int)i);
-                if (__any(sw)) {
-                    sfor<0, N>([&](auto t) {
-                        const double a = A[k][t], c = A[i][t];
-                        A[k][t] = sw ? c : a;
-                        A[i][t] = sw ? a : c;
-                    });
-                    const double a = s[k], c = s[i];
-                    s[k] = sw ? c : a;
-                    s[i] = sw ? a : c;
-                    const double u = b[k], v = b[i];
-                    b[k] = sw ? v : u;
-                    b[i] = sw ? u : v;
-                }
-            });
+        if constexpr (k + 1 < N) {
+            double mo = 0.0;
+            sfor<k + 1, N - 1>([&](auto i) { mo = fmax(mo, fabs(A[i][k])); });
+            const bool want = 0.1 * mo > fabs(A[k][k]) || A[k][k] == 0.0;
+            if (__any(want)) {
+                int ik = k;
+                double maxs = want ? fabs(A[k][k]) : __builtin_huge_val();
+                sfor<k + 1, N>([&](auto i) {
+                    const bool g = i < N - 1 ? fabs(A[i][k]) > maxs : maxs == 0.0;
+                    ik = g ? (int)i : ik;
+                    maxs = g ? fabs(A[i][k]) : maxs;
+                });
+                sfor<k + 1, N>([&](auto i) {
+                    const bool sw = (ik == (int)i);
+                    if (__any(sw)) {
+                        sfor<k, N>([&](auto t) {
+                            const double a = A[k][t], c = A[i][t];
+                            A[k][t] = sw ? c : a;
+                            A[i][t] = sw ? a : c;
+                        });
+                        const double u = b[k], v = b[i];
+                        b[k] = sw ? v : u;
+                        b[i] = sw ? u : v;
+                    }
+                });
+            }
         }
-        A[k][k] = s[k];
-        sfor<k + 1, N>([&](auto j) {
-            double sum = 0.0;
-            sfor<0, k>([&](auto t) { sum += A[k][t] * A[t][j]; });
-            A[k][j] -= sum;
-        });
         dinv[k] = frcp(A[k][k]);
-        sfor<k + 1, N>([&](auto i) { A[i][k] = s[i] * dinv[k]; });
-    });
-    sfor<0, N>([&](auto i) {
-        double sum = 0.0;
-        sfor<0, i>([&](auto t) { sum += A[i][t] * b[t]; });
-        b[i] -= sum;
+        sfor<k + 1, N>([&](auto i) {
+            const double l = -A[i][k] * dinv[k];
+            sfor<k + 1, N>([&](auto j) { A[i][j] = fma(l, A[k][j], A[i][j]); });
+            b[i] = fma(l, b[k], b[i]);
+        });
     });
     sfor<0, N>([&](auto ii) {
         constexpr int i = N - 1 - ii;
-        double sum = 0.0;
-        sfor<i + 1, N>([&](auto t) { sum += A[i][t] * b[t]; });
-        b[i] = (b[i] - sum) * dinv[i];
+        b[i] *= dinv[i];
+        sfor<0, i>([&](auto t) { b[t] = fma(-A[t][i], b[i], b[t]); });
     });
 }
 

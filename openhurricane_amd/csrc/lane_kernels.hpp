@@ -102,6 +102,8 @@ __global__ __launch_bounds__(64) void ie_lane_kernel(const LaneParams P) {
     enum { Q_ATOL, Q_RTOL, Q_ATOLI, Q_RTOLI, Q_SAFE, Q_MINSC, Q_MAXSC, Q_ALPHA, Q_TTHR, Q_TALPHA,
            Q_TBETA, Q_DTMAX, Q_DTF, Q_ERRG, Q_NPAR };
     __shared__ double s_par[Q_NPAR];
+    __shared__ __attribute__((aligned(16))) double s_th[ThermoTab<M>::kSize];
+    for (int i = lane; i < ThermoTab<M>::kSize; i += 64) s_th[i] = kThermoTab<M>.v[i];
     if (lane == 0) {
         s_par[Q_ATOL] = P.atol;
         s_par[Q_RTOL] = P.rtol;
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(64) void ie_lane_kernel(const LaneParams P) {
             double yk[N];
 #pragma unroll
             for (int i = 0; i < N; ++i) yk[i] = YK(i);
-            eval_fJ<M, true, FLOW, F, true>(yk, pr, f, J, P.exact_dkp != 0);
+            eval_fJ<M, true, FLOW, F, true>(yk, pr, f, J, P.exact_dkp != 0, s_th);
         }
 
         bool have = false;
@@ -398,13 +400,14 @@ __global__ __launch_bounds__(64) void ie_lane_kernel(const LaneParams P) {
             aerr = max_increment(f);
         }
         if (__any(phase == PH_NEWTON)) {
-            // (I - dt J) delta = -yk + y0 + dt f  (ImplicitEuler.cpp:186-198)
+            // (I - dt J) delta = -yk + y0 + dt f  (ImplicitEuler.cpp:186-198),
+            // divided by -dt: only the diagonal of J changes (dt = 0: no update)
             const double h = TR ? 0.5 * dtl : dtl;
+            const double rh = fabs(h) < 1e-300 ? 1e300 : frcp(h);
             sfor<0, N>([&](auto i) {
-                sfor<0, N>([&](auto j) { J[i][j] = -h * J[i][j]; });
-                J[i][i] += 1.0;
-                if constexpr (TR) f[i] = -YK(i) + Y0(i) + h * (F0(i) + f[i]);
-                else f[i] = -YK(i) + Y0(i) + h * f[i];
+                J[i][i] -= rh;
+                if constexpr (TR) f[i] = (YK(i) - Y0(i)) * rh - (F0(i) + f[i]);
+                else f[i] = (YK(i) - Y0(i)) * rh - f[i];
             });
             lu_solve<N>(J, f);
         }

@@ -96,3 +96,38 @@ def test_cells_without_a_number_fail_and_leave_the_others(h2mech):
     if np.isfinite(Tb[keep]).all() and not np.array_equal(Tb, st["T"]):
         np.testing.assert_array_equal(Tb[keep], T[keep])
         np.testing.assert_array_equal(Yb[:, keep], Y[:, keep])
+
+
+@pytest.mark.parametrize("integrator,n", [(2, 67), (0, (1 << 17) + 5)])
+@pytest.mark.parametrize("flow", [0, 1])
+def test_lane_kernel_outside_the_fits(h2mech, h2oracle, integrator, n, flow):
+    """One cell per lane at temperatures below, inside and above the thermo fits
+    (clamped there), in one wavefront; cells inside keep their bits whatever
+    their neighbours are."""
+    from openhurricane_amd.chemistry import ChemistrySource
+
+    o = _opts(flow_type=flow, integrator=integrator, T_threshold=100.0)
+    cs = ChemistrySource(h2mech, opts=o)
+    m = 67
+    st = _states(h2mech, m, 33)
+    lo, hi = h2mech.tables()["Tlow"].max(), h2mech.tables()["Thigh"].min()
+    Tx = st["T"].copy()
+    Tx[::5] = lo - 40.0
+    Tx[3::11] = hi + 60.0
+    out = (Tx < lo) | (Tx > hi)
+    assert 0 < out.sum() < m
+    idx = np.arange(n) % m
+    res = {}
+    for name, T0 in (("mixed", Tx), ("inside", st["T"])):
+        print(f"integrator {integrator}, {n} cells, {name}", flush=True)
+        T, Y = T0[idx].copy(), np.ascontiguousarray(st["Y"][:, idx])
+        rho = np.ascontiguousarray((st["rho"] * st["T"] / T0)[idx])
+        cs.solve_update(T, np.ascontiguousarray(st["p"][idx]), rho, Y, np.full(n, 1e-8), 1.0)
+        res[name] = (T, Y)
+    np.testing.assert_array_equal(res["mixed"][0][~out[idx]], res["inside"][0][~out[idx]])
+    np.testing.assert_array_equal(res["mixed"][1][:, ~out[idx]], res["inside"][1][:, ~out[idx]])
+    To, Yo, _, _ = h2oracle.solve_update(o, Tx, st["p"], st["rho"] * st["T"] / Tx, st["Y"],
+                                         np.full(m, 1e-8), 1.0)
+    T, Y = res["mixed"][0][:m], res["mixed"][1][:, :m]
+    assert (np.abs(T - To) / To).max() <= 1e-6
+    assert (np.abs(Y - Yo) / np.maximum(Yo, 1e-3)).max() <= 1e-6
