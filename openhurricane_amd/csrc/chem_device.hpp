@@ -107,6 +107,38 @@ __device__ __forceinline__ double frcp(double x) {
     return fma(e, r, r);
 }
 
+// 1/x without frcp's zero and infinity cases (those come out NaN)
+__device__ __forceinline__ double rcp_raw(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+// ln x to a few 1e-16 of max(1, |ln x|), x held to [1e-290, 1e290]: mantissa m in
+// [sqrt(1/2), sqrt(2)), s = (m - 1) / (m + 1), the series of 2 artanh(s); half the
+// library logarithm's dependent chain and no branch.
+__device__ __forceinline__ double log_pos(double x) {
+    x = fmin(fmax(x, 1.0e-290), 1.0e290);
+    double m = __builtin_amdgcn_frexp_mant(x);
+    int e = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    e -= low ? 1 : 0;
+    const double s = (m - 1.0) * rcp_raw(m + 1.0), z = s * s, y = z * z;
+    // even and odd powers apart: two shorter chains
+    double p = 2.0 / 21.0, q = 2.0 / 19.0;
+    p = fma(p, y, 2.0 / 17.0);
+    q = fma(q, y, 2.0 / 15.0);
+    p = fma(p, y, 2.0 / 13.0);
+    q = fma(q, y, 2.0 / 11.0);
+    p = fma(p, y, 2.0 / 9.0);
+    q = fma(q, y, 2.0 / 7.0);
+    p = fma(p, y, 2.0 / 5.0);
+    q = fma(q, y, 2.0 / 3.0);
+    p = fma(p, y, 2.0);
+    return fma((double)e, 0.69314718055994530942, s * fma(q, z, p));
+}
+
 // refined 1/sqrt(x), x normal and positive
 __device__ __forceinline__ double frsq(double x) {
     double r = __builtin_amdgcn_rsq(x);
@@ -298,13 +330,12 @@ __device__ __forceinline__ void thermo_pairs(const double *tab, double T, double
     }
 }
 
-// species_G on the table; OUT: some lane is outside the fits (a lane inside gets
-// the same bits either way).  Inside, cp0 and T ds0/dT are the same polynomial.
+// species_G on pairs 0..5 of the table (c); OUT: some lane is outside the fits (a
+// lane inside gets the same bits either way).  Inside, cp0 and T ds0/dT are the
+// same polynomial.
 template <class M, int k, bool OUT>
-__device__ __forceinline__ void species_G_tab(const double *tab, double T, double lnT, double &G,
-                                              double &dG) {
-    double c[12];
-    thermo_pairs<M, k, 0, 6>(tab, T, c);
+__device__ __forceinline__ void species_G_tab(const double (&c)[12], const double *tab, double T,
+                                              double lnT, double &G, double &dG) {
     const double s0 = fma(fma(fma(fma(c[0], T, c[1]), T, c[2]), T, c[3]), T, fma(c[4], lnT, c[5]));
     const double g0 = fma(fma(fma(c[6], T, c[7]), T, c[8]), T, c[9]);
     G = fma(fma(g0, T, fma(c[4], 1.0 - lnT, -c[5])), T, c[10]);
@@ -321,12 +352,10 @@ __device__ __forceinline__ void species_G_tab(const double *tab, double T, doubl
     }
 }
 
-// species_CH on the table
+// species_CH on pairs 6..12 of the table (c)
 template <class M, int k, bool OUT>
-__device__ __forceinline__ void species_CH_tab(const double *tab, double T, double &Cp, double &H,
-                                               double &dCp) {
-    double c[14];
-    thermo_pairs<M, k, ThermoTab<M>::T_C / 2, 7>(tab, T, c);
+__device__ __forceinline__ void species_CH_tab(const double (&c)[14], double T, double &Cp,
+                                               double &H, double &dCp) {
     double Tx = T;
     if constexpr (OUT) {
         const double Tl = M::Tlow[k], Th = M::Thigh[k];
@@ -548,9 +577,12 @@ struct MSumS {
 // Equilibrium terms of reversible reaction r: Kc, rK = 1/max(Kc, veryTiny)
 // and (optionally) dKc/dT -- reactionTypes.cpp:178-241 (dKp/dT with the
 // reference's sign convention).
-template <class M, int r, bool WITH_D, class F = double>
+// GUARD = false leaves out the limits of Kp, Kc and their derivatives: right if
+// lim, to which Kp + 1/Kp is added, stays below kGuardLim and dKc/dT is finite.
+constexpr double kGuardLim = 1.0e100;
+template <class M, int r, bool WITH_D, bool GUARD, class F = double>
 __device__ __forceinline__ void equilibrium(const TFac &tf, const Thermo<M> &th, double &Kc,
-                                            double &rK, double &dKc, bool exact) {
+                                            double &rK, double &dKc, bool exact, double &lim) {
     constexpr RxnD d = M::R[r];
     constexpr bool zero_s = cabs(d.sumStoi) < kVeryTiny;
     constexpr bool kc_species = M::KC_SPECIES && std::is_same_v<F, double>;
@@ -590,7 +622,9 @@ __device__ __forceinline__ void equilibrium(const TFac &tf, const Thermo<M> &th,
             sfor<0, d.nf>([&](auto i) { dk -= th.dG[d.fi[i]] * d.fnu[i]; });
             sfor<0, d.nb>([&](auto i) { dk += th.dG[d.bi[i]] * d.bnu[i]; });
         }
-        if (bad(Kp)) {
+        if constexpr (!GUARD) {
+            lim += Kp + rKp;
+        } else if (bad(Kp)) {
             Kp = kRootVeryLarge;
             rKp = 1.0 / kRootVeryLarge;
         }
@@ -620,7 +654,11 @@ __device__ __forceinline__ void equilibrium(const TFac &tf, const Thermo<M> &th,
         Xs = Xpow<SumS<M, r>>(tf);
         Kc = fmin(Kp * Xs, kVeryLarge);
     }
-    if constexpr (kc_species) {
+    if constexpr (!GUARD) {
+        Kc = 1.0;  // not below the limits
+        if constexpr (zero_s) rK = rKp;
+        else rK = rKp * Xpow<MSumS<M, r>>(tf);
+    } else if constexpr (kc_species) {
         double rKc = rKp;
         if constexpr (!zero_s) rKc = Kc == kVeryLarge ? 1.0 / kVeryLarge : rKp * Xpow<MSumS<M, r>>(tf);
         rK = Kc > kVeryTiny ? rKc : 1.0 / kVeryTiny;
@@ -629,12 +667,13 @@ __device__ __forceinline__ void equilibrium(const TFac &tf, const Thermo<M> &th,
     }
     if constexpr (WITH_D) {
         if (exact) dk = -dk;  // exact d(Kp)/dT = -Kp d(sum nu G/(Ru T))/dT
+        // (fma written out: the same rounding with and without the limits)
         double dKp = Kp * dk;
-        if (bad(dKp)) dKp = kVeryLarge;
+        if (GUARD && bad(dKp)) dKp = kVeryLarge;
         if constexpr (zero_s) dKc = dKp;
         else {
-            double v = (dKp + Kp * (-d.sumStoi) * tf.invT) * Xs;
-            if (bad(v)) v = kVeryLarge;
+            double v = fma(Kp * -d.sumStoi, tf.invT, dKp) * Xs;
+            if (GUARD && bad(v)) v = kVeryLarge;
             dKc = v;
         }
     } else {
@@ -698,6 +737,15 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
     constexpr bool fp32 = std::is_same_v<F, float>;
     constexpr bool TAB = UNI && !fp32 && ThermoTab<M>::kFits;
     const double T = y[NS];
+    // all coefficients of G are on their way while the logarithm and the
+    // reciprocals are computed, those of Cp and H two species ahead: the one
+    // wavefront of a SIMD has nothing else to do while it waits (192 -> 187 ms for
+    // 1,048,576 H2-air cells)
+    double cG[TAB ? NS : 1][12];
+    if constexpr (TAB) {
+        sfor<0, NS>([&](auto k) { thermo_pairs<M, k, 0, 6>(tab, T, cG[k]); });
+        __builtin_amdgcn_sched_barrier(0);
+    }
     const TFac tf = tfac(T);
     const bool hi = UNI && !TAB && wave_all_high<M>(T);
     const bool out = TAB && __any(T < tlow_max<M>() || T > thigh_min<M>());
@@ -706,7 +754,7 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
         constexpr int R = decltype(Rc)::value;
         sfor<0, NS>([&](auto k) {
             if constexpr (TAB)
-                species_G_tab<M, k, R != 0>(tab, T, tf.lnT, th.G[k], th.dG[k]);
+                species_G_tab<M, k, R != 0>(cG[k], tab, T, tf.lnT, th.G[k], th.dG[k]);
             else if constexpr (fp32)
                 species_G32<M, k, R>(T, (float)tf.lnT, (float)tf.invTm, th.G[k], th.dG[k]);
             else
@@ -732,8 +780,12 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
     sfor<0, M::NTB>([&](auto g) {
         Mg[g] = third_M<M, g>(ci);
         rMg[g] = 1.0 / fmax(Mg[g], kTiny);
-        sfor<0, NS>([&](auto a) { u[g][a] = 0.0; });
     });
+    double lim = 0.0;
+    auto react = [&](auto guard, const TFac &tf, const Thermo<M> &th, const double(&ci)[NS])
+                     __attribute__((always_inline)) {
+    constexpr bool GUARD = decltype(guard)::value;
+    sfor<0, M::NTB>([&](auto g) { sfor<0, NS>([&](auto a) { u[g][a] = 0.0; }); });
     sfor<0, N>([&](auto i) {
         f[i] = 0.0;
         if constexpr (WITH_J) sfor<0, N>([&](auto j) { J[i][j] = 0.0; });
@@ -755,7 +807,7 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
             else kf = fo.k0 * (1.0 / (1.0 + fo.Pr)) * fo.F;
         }
         if constexpr (d.rev == 1) {
-            equilibrium<M, r, WITH_J, F>(tf, th, Kc, rKc, dKc, exact);
+            equilibrium<M, r, WITH_J, GUARD, F>(tf, th, Kc, rKc, dKc, exact, lim);
             kr = Kc > kVeryTiny ? kf * rKc : 0.0;
         } else if constexpr (d.rev == 2) {
             kr = arrh<2, R, F>(tf.lnT, tf.invT);
@@ -851,13 +903,45 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
                     dgdT = q * gg;
                 }
             }
-            if (bad(dqdT)) dqdT = 0.0;
+            if (GUARD && bad(dqdT)) dqdT = 0.0;
             if (bad(dgdT)) dgdT = 0.0;
             const double s = dqdT + dgdT;
             sfor<0, d.nf>([&](auto i) { J[d.fi[i]][NS] -= d.fnu[i] * s; });
             sfor<0, d.nb>([&](auto i) { J[d.bi[i]][NS] += d.bnu[i] * s; });
         }
     });
+    };
+    // the limits of the equilibrium constants and the tests for overflow (25 of
+    // some 90 instructions of a reversible reaction) only where a lane needs them:
+    // 203 -> 192 ms for 1,048,576 H2-air cells
+    if constexpr (WITH_J && UNI && !fp32 && M::KC_SPECIES) {
+        react(std::false_type{}, tf, th, ci);
+        sfor<0, NS>([&](auto i) { lim = fma(J[i][NS], 0.0, lim); });
+        if (__any(!(lim < kGuardLim))) {
+            // from copies the compiler cannot see through, or it would keep every
+            // value that both passes compute alive across this branch
+            TFac tg = tf;
+            Thermo<M> tc;
+            double cc[NS];
+            auto hide = [](double x) {
+                asm volatile("" : "+v"(x));
+                return x;
+            };
+            tg.lnT = hide(tf.lnT);
+            tg.invT = hide(tf.invT);
+            tg.invTm = hide(tf.invTm);
+            tg.invRuT = hide(tf.invRuT);
+            sfor<0, NS>([&](auto k) {
+                tc.G[k] = hide(th.G[k]);
+                tc.H[k] = hide(th.H[k]);
+                tc.dG[k] = hide(th.dG[k]);
+                cc[k] = hide(ci[k]);
+            });
+            react(std::true_type{}, tg, tc, cc);
+        }
+    } else {
+        react(std::true_type{}, tf, th, ci);
+    }
     if constexpr (WITH_J && !MA) {
         sfor<0, M::NTB>([&](auto g) {
             sfor<0, NS>([&](auto a) {
@@ -874,8 +958,19 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
     // ---- temperature row (chemistrySource.cpp:993-1020 / :1021-1054)
     auto cph = [&](auto Rc) {
         constexpr int R = decltype(Rc)::value;
+        constexpr int kAhead = 2;
+        double c[kAhead + 1][14];
+        auto load = [&](auto k) {
+            if constexpr (TAB && k < NS)
+                thermo_pairs<M, k, ThermoTab<M>::T_C / 2, 7>(tab, T, c[k % (kAhead + 1)]);
+        };
+        sfor<0, kAhead>(load);
         sfor<0, NS>([&](auto k) {
-            if constexpr (TAB) species_CH_tab<M, k, R != 0>(tab, T, th.Cp[k], th.H[k], th.dCp[k]);
+            if constexpr (TAB) {
+                load(std::integral_constant<int, k + kAhead>{});
+                __builtin_amdgcn_sched_barrier(0);
+                species_CH_tab<M, k, R != 0>(c[k % (kAhead + 1)], T, th.Cp[k], th.H[k], th.dCp[k]);
+            }
             else species_CH<M, k>(Coef<M, k, R>(T), T, th.Cp[k], th.H[k], th.dCp[k]);
         });
     };
@@ -927,7 +1022,7 @@ __device__ __forceinline__ void eval_fJ(const double (&y)[M::NS + 1], double pr,
 // are done with selects and skipped when no lane of the wavefront needs them.
 // Exchanging for every larger entry (the temperature row's among them) cost the
 // integrator of 1,048,576 H2-air cells 239 ms a step; with a species row's tenth
-// 232, with the thermo table and this form 203.
+// 232, in this form with the thermo table 203.
 template <int N>
 __device__ __forceinline__ void lu_solve(double (&A)[N][N], double (&b)[N]) {
     double dinv[N];

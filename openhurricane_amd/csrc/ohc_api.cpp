@@ -367,9 +367,10 @@ void base_params(const ohc_ctx *c, ohcd::LaneParams &P) {
 
 // Calls of up to this many cells run four cells per wavefront on compiled
 // mechanisms (quad_lane.hpp): beyond, the time is that of the work, which one
-// lane per cell does in a quarter of the instructions.  131,072 H2-air cells take
-// 210 ms here and 264 ms there, 262,144 366 and 275.
-constexpr int64_t kQuadLaneMax = 1 << 17;
+// lane per cell does in a fifth of the instructions.  98,304 H2-air cells take
+// 170 ms here and 172 there (113 and 165 with the sub-steps of the step before),
+// 131,072 210 and 172 (151 and 165).
+constexpr int64_t kQuadLaneMax = 3 << 15;
 
 // Cells that a wavefront of the integrator holds at a time in a call of n cells.
 static int cells_per_wave(const ohc_ctx *c, int64_t n) {

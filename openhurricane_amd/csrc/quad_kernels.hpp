@@ -92,38 +92,6 @@ __device__ __forceinline__ double gmax(double v) {
 __device__ __forceinline__ bool gany(bool x) {
     return ((__builtin_amdgcn_ballot_w64(x) >> (threadIdx.x & 48u)) & 0xffffull) != 0ull;
 }
-// 1/x without frcp's zero and infinity cases (those come out NaN, which the
-// backward-error check turns away)
-__device__ __forceinline__ double rcp_raw(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
-}
-
-// ln x to a few 1e-16 of max(1, |ln x|), x held to [1e-290, 1e290]: mantissa m in
-// [sqrt(1/2), sqrt(2)), s = (m - 1) / (m + 1), the series of 2 artanh(s); half the
-// library logarithm's dependent chain and no branch.
-__device__ __forceinline__ double log_pos(double x) {
-    x = fmin(fmax(x, 1.0e-290), 1.0e290);
-    double m = __builtin_amdgcn_frexp_mant(x);
-    int e = __builtin_amdgcn_frexp_exp(x);
-    const bool low = m < 0.70710678118654752;
-    m = low ? m + m : m;
-    e -= low ? 1 : 0;
-    const double s = (m - 1.0) * rcp_raw(m + 1.0), z = s * s, y = z * z;
-    // even and odd powers apart: two shorter chains
-    double p = 2.0 / 21.0, q = 2.0 / 19.0;
-    p = fma(p, y, 2.0 / 17.0);
-    q = fma(q, y, 2.0 / 15.0);
-    p = fma(p, y, 2.0 / 13.0);
-    q = fma(q, y, 2.0 / 11.0);
-    p = fma(p, y, 2.0 / 9.0);
-    q = fma(q, y, 2.0 / 7.0);
-    p = fma(p, y, 2.0 / 5.0);
-    q = fma(q, y, 2.0 / 3.0);
-    p = fma(p, y, 2.0);
-    return fma((double)e, 0.69314718055994530942, s * fma(q, z, p));
-}
 
 // What the Newton system needs of one evaluation, besides J in LDS.
 template <int S>

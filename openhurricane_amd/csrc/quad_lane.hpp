@@ -3,8 +3,8 @@
 // do not fill the chip with one cell per lane.
 //
 // One lane per cell gives the best throughput, but a Newton iteration of a
-// wavefront then takes 14 us, and a stiff H2-air cell needs 17,000 of them: a
-// call of 64 cells and one of 65,536 both took as long as their slowest cell.
+// wavefront then takes 10 us, and a stiff H2-air cell needs 17,000 of them: a
+// call of 64 cells and one of 65,536 both take as long as their slowest cell.
 // With 16 lanes per cell an iteration is spread over the lanes -- species k and row
 // k of the Newton matrix in lane k, reactions r and r + 16 in lane r -- and takes
 // about 2 us.  Nothing but the concentrations goes through LDS:
@@ -20,10 +20,9 @@
 // step control 4,000), so the kernel takes all registers of a SIMD: with two
 // wavefronts per SIMD and half the registers 64 cells took 71 ms for 60.
 //
-// Measured, one flow step of stiff H2-air, one lane per cell -> here: 64 cells
-// 212 -> 60 ms, 1,000 242 -> 73, 65,536 264 -> 132 (with the sub-steps of the step
-// before 235 -> 80), 131,072 264 -> 210 (236 -> 151), 262,144 275 -> 366 (238 ->
-// 305).
+// Measured, one flow step of stiff H2-air, one lane per cell -> here, ms: 64
+// cells 150 -> 60, 65,536 172 -> 132 (with the sub-steps of the step before 165 ->
+// 80), 98,304 172 -> 170 (165 -> 113), 131,072 172 -> 210 (165 -> 151).
 #pragma once
 
 #include "quad_kernels.hpp"

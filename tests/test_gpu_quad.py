@@ -131,3 +131,51 @@ def test_lane_kernel_outside_the_fits(h2mech, h2oracle, integrator, n, flow):
     T, Y = res["mixed"][0][:m], res["mixed"][1][:, :m]
     assert (np.abs(T - To) / To).max() <= 1e-6
     assert (np.abs(Y - Yo) / np.maximum(Yo, 1e-3)).max() <= 1e-6
+
+
+@pytest.mark.parametrize("flow", [0, 1])
+def test_compiled_limit_agrees(h2mech, flow):
+    """98,304 and 98,305 cells: four cells per wavefront and one cell per lane."""
+    from openhurricane_amd.chemistry import ChemistrySource
+
+    cs = ChemistrySource(h2mech, opts=_opts(flow_type=flow))
+    m, res = 500, []
+    st = _states(h2mech, m, 22)
+    for n in (3 << 15, (3 << 15) + 1):
+        print(f"{n} cells", flush=True)
+        idx = np.arange(n) % m
+        T, Y = st["T"][idx], np.ascontiguousarray(st["Y"][:, idx])
+        sub, s = cs.solve_update(T, np.ascontiguousarray(st["p"][idx]),
+                                 np.ascontiguousarray(st["rho"][idx]), Y, np.full(n, 1e-7), 1.0)
+        np.testing.assert_array_equal(T, T[:m][idx])
+        res.append((T[:m], Y[:, :m], sub[:m], s["steps"] / n))
+    np.testing.assert_allclose(res[1][0], res[0][0], rtol=1e-9)
+    np.testing.assert_allclose(res[1][1], res[0][1], rtol=1e-9, atol=1e-12)
+    np.testing.assert_allclose(res[1][2], res[0][2], rtol=1e-9)
+    assert abs(res[1][3] - res[0][3]) <= 0.01 * res[0][3]
+
+
+def test_cold_neighbours_take_the_guarded_pass(h2mech):
+    """A wavefront in which one cell's equilibrium constants pass 1e100 (150 K)
+    evaluates the reactions with all limits; the other cells keep their bits."""
+    from openhurricane_amd.chemistry import ChemistrySource
+
+    cs = ChemistrySource(h2mech, opts=_opts(T_threshold=100.0))
+    n, m = (1 << 17) + 64, 64
+    st = _states(h2mech, m, 41)
+    idx = np.arange(n) % m
+    res = []
+    for cold in (False, True):
+        T0 = st["T"].copy()
+        if cold:
+            T0[7] = 150.0
+        T, Y = T0[idx], np.ascontiguousarray(st["Y"][:, idx])
+        print("cold", cold, flush=True)
+        cs.solve_update(T, np.ascontiguousarray(st["p"][idx]),
+                        np.ascontiguousarray((st["rho"] * st["T"] / T0)[idx]), Y,
+                        np.full(n, 1e-8), 1.0)
+        assert np.isfinite(T).all() and np.isfinite(Y).all()
+        res.append((T, Y))
+    keep = idx != 7
+    np.testing.assert_array_equal(res[1][0][keep], res[0][0][keep])
+    np.testing.assert_array_equal(res[1][1][:, keep], res[0][1][:, keep])
