@@ -7,7 +7,7 @@
 // call of 64 cells and one of 65,536 both take as long as their slowest cell.
 // With 16 lanes per cell an iteration is spread over the lanes -- species k and row
 // k of the Newton matrix in lane k, reactions r and r + 16 in lane r -- and takes
-// about 2 us.  Nothing but the concentrations goes through LDS:
+// about 3.5 us.  Nothing but the concentrations goes through LDS:
 //   * a reaction lane evaluates its rate constant, the equilibrium constant from
 //     the reaction's own summed NASA-7 coefficients, and the partial derivatives
 //     of its net rate;
